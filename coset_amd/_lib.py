@@ -95,6 +95,7 @@ OPT_CODEC_PLAIN = 5
 OPT_CODEC_DYNAMIC = 6
 OPT_VLUT_DEEP = 7
 OPT_GEMM_TN_TILE = 8
+OPT_VLUT_GEMM = 9
 CODEC_AUTO, CODEC_GENERIC, CODEC_LUT = 0, 1, 2
 
 _lib = None
@@ -214,6 +215,13 @@ def set_vlut_decode(byte_tables: bool) -> None:
 def set_vlut_deep(enabled: bool) -> None:
     """vLUT matmuls above 32 tokens: the deep kernel (default) or the wide one."""
     call("coset_set_option", OPT_VLUT_DEEP, int(bool(enabled)))
+
+
+def set_vlut_gemm(mode: int) -> None:
+    """Large vLUT batches of the decoded formats: 0 the deep kernel, 1 the
+    GEMM kernel where the plan prefers it (default), 2 + s its tile shape s
+    (256 x 256, 256 x 192, 128 x 128 or 128 x 64 tokens x rows) always."""
+    call("coset_set_option", OPT_VLUT_GEMM, int(mode))
 
 
 def set_gemm_tn_tile(tile: int) -> None:

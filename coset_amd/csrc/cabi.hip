@@ -127,6 +127,10 @@ int coset_set_option(int key, int value)
         if (value < 0 || value > 1) return fail(COSET_EINVAL, "vLUT deep %d not in {0,1}", value);
         coset::g_vlut_deep = value;
         return COSET_OK;
+    case COSET_OPT_VLUT_GEMM:
+        if (value < 0 || value > 5) return fail(COSET_EINVAL, "vLUT gemm %d not in 0..5", value);
+        coset::g_vlut_gemm = value;
+        return COSET_OK;
     case COSET_OPT_GEMM_TN_TILE:
         if (value != 0 && value != 64 && value != 96) return fail(COSET_EINVAL, "gemm_tn tile %d not in {0,64,96}", value);
         coset::g_gemm_tn_tile = value;
@@ -752,7 +756,8 @@ static int vlut_matmul_impl(const void* words, int word_format, const float* sca
     if (!aligned(act, 16) || !aligned(words, 4)) return fail(COSET_EINVAL, "act must be 16-byte aligned, words 4-byte");
     const bool split = m == coset::VLUT_METHOD_MFMA_SPLIT;
     // the split path's inner product: 3B bf16 tokens on the matrix cores
-    const coset::VlutPlan plan = coset::vlut_plan(rows, split ? 3 * B : B, K, q, M, split ? coset::VLUT_METHOD_MFMA : m);
+    const coset::VlutPlan plan = coset::vlut_plan(rows, split ? 3 * B : B, K, q, M, split ? coset::VLUT_METHOD_MFMA : m,
+                                                   word_format);
     const int64_t need = vlut_method_workspace(m, B, rows, K, q, M);
     if (workspace_floats < need)
         return fail(COSET_EINVAL, "workspace holds %lld floats, needs %lld", (long long)workspace_floats,
@@ -760,9 +765,10 @@ static int vlut_matmul_impl(const void* words, int word_format, const float* sca
     if (need > 0 && !workspace) return fail(COSET_EINVAL, "NULL workspace");
     if (word_format < 0 || word_format > 5) return fail(COSET_EINVAL, "word_format must be 0, 1, 2, 3, 4 or 5");
     if (word_format == 3 && plan.kernel != coset::VK_MFMA_ROWS && plan.kernel != coset::VK_MFMA_WIDE &&
-        plan.kernel != coset::VK_MFMA_DEEP)
+        plan.kernel != coset::VK_MFMA_DEEP && plan.kernel != coset::VK_MFMA_GEMM)
         return fail(COSET_EUNSUPPORTED, "the decoded format runs on the matrix-core rows kernel only (fp16/bf16 activations)");
-    if (word_format == 5 && plan.kernel != coset::VK_MFMA_ROWS && plan.kernel != coset::VK_MFMA_DEEP)
+    if (word_format == 5 && plan.kernel != coset::VK_MFMA_ROWS && plan.kernel != coset::VK_MFMA_DEEP &&
+        plan.kernel != coset::VK_MFMA_GEMM)
         return fail(COSET_EUNSUPPORTED, "the 6-byte decoded format runs on the matrix-core rows and deep kernels only");
     if (word_format != 0 && !aligned(words, 16)) return fail(COSET_EINVAL, "prepared words must be 16-byte aligned");
     coset::VlutMatmulArgs p{};

@@ -911,6 +911,7 @@ hipError_t vlut_dot(const void* words, int64_t n, int M, int q, const float* vlu
 int g_vlut_swar = 1;
 int g_vlut_splits = 0;
 int g_vlut_deep = 1;
+int g_vlut_gemm = 1;
 
 namespace {
 
@@ -929,7 +930,7 @@ int device_cu_count()
 
 }  // namespace
 
-VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method)
+VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method, int fmt)
 {
     const int64_t kb = K / 8;
     if (method == VLUT_METHOD_LDS) {
@@ -939,9 +940,14 @@ VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method)
         const int64_t groups = ((rows + lds_rows(B) - 1) / lds_rows(B)) * ((B + TT - 1) / TT);
         int64_t splits = g_vlut_splits > 0 ? g_vlut_splits
                                            : (2 * device_cu_count() + groups - 1) / std::max<int64_t>(1, groups);
-        return {VK_LDS, (int)std::max<int64_t>(1, std::min<int64_t>(splits, kb))};
+        return {VK_LDS, (int)std::max<int64_t>(1, std::min<int64_t>(splits, kb)), 0};
     }
     const bool swar = g_vlut_swar && ((q == 2 && M <= 4) || (q == 4 && M <= 2));
+    if (swar && g_vlut_deep && g_vlut_gemm && g_vlut_splits == 0 &&
+        (fmt == VLUT_DECODED || fmt == VLUT_DECODED6)) {
+        const int shape = g_vlut_gemm >= 2 ? g_vlut_gemm - 2 : vlut_gemm_shape(rows, B, K, device_cu_count());
+        if (shape >= 0) return {VK_MFMA_GEMM, 1, shape};
+    }
     if (swar && B > 32 && g_vlut_deep) {
         // 64-row, 64-token workgroups, at most 32 k-quads each: enough K
         // splits for that, and more (down to one k-quad per workgroup) to
@@ -952,7 +958,7 @@ VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method)
         int64_t splits = g_vlut_splits > 0 ? g_vlut_splits
                                            : std::max<int64_t>(1, device_cu_count() / std::max<int64_t>(1, groups));
         splits = std::max(min_splits, std::min<int64_t>(splits, kq_total));
-        return {VK_MFMA_DEEP, (int)splits};
+        return {VK_MFMA_DEEP, (int)splits, 0};
     }
     if (swar && B > 32) {
         // 128-row, 64-token workgroups sharing the activations through LDS,
@@ -961,7 +967,7 @@ VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method)
         const int64_t max_splits = std::max<int64_t>(1, ((kb + 3) / 4) / kWideStageKq);
         int64_t splits = g_vlut_splits > 0 ? g_vlut_splits
                                            : std::max<int64_t>(1, device_cu_count() / std::max<int64_t>(1, groups));
-        return {VK_MFMA_WIDE, (int)std::max<int64_t>(1, std::min<int64_t>(splits, max_splits))};
+        return {VK_MFMA_WIDE, (int)std::max<int64_t>(1, std::min<int64_t>(splits, max_splits)), 0};
     }
     if (swar) {
         // one workgroup of 16 rows per CU when the rows allow, else K splits
@@ -970,7 +976,7 @@ VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method)
         const int64_t max_splits = std::max<int64_t>(1, ((kb + 3) / 4) / kRowsWaves);
         int64_t splits = g_vlut_splits > 0 ? g_vlut_splits
                                            : (device_cu_count() + row_tiles - 1) / std::max<int64_t>(1, row_tiles);
-        return {VK_MFMA_ROWS, (int)std::max<int64_t>(1, std::min<int64_t>(splits, max_splits))};
+        return {VK_MFMA_ROWS, (int)std::max<int64_t>(1, std::min<int64_t>(splits, max_splits)), 0};
     }
     // every workgroup covers at most kMfmaMaxSteps * 16 k-blocks; beyond
     // that minimum, small batches take more splits (more workgroups in
@@ -981,7 +987,7 @@ VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method)
     int64_t want = B <= 16 ? 2048 : 512;
     int64_t splits = g_vlut_splits > 0 ? g_vlut_splits
                                        : std::max<int64_t>(min_splits, want / std::max<int64_t>(1, row_tiles));
-    return {VK_MFMA_TILE, (int)std::max<int64_t>(1, std::min<int64_t>(std::max(splits, min_splits), max_splits))};
+    return {VK_MFMA_TILE, (int)std::max<int64_t>(1, std::min<int64_t>(std::max(splits, min_splits), max_splits)), 0};
 }
 
 // One tile entry (pair) per thread: 2 x_hat = sum_m q^m 2 r(b_m) with the
@@ -1168,7 +1174,7 @@ hipError_t vlut_matmul_split(VlutMatmulArgs p, float* workspace, hipStream_t s)
     q.act_dtype = DT_BF16;
     q.B = 3 * B;
     q.partial = inner;
-    const VlutPlan plan = vlut_plan(p.rows, 3 * B, p.K, p.q, p.M, VLUT_METHOD_MFMA);
+    const VlutPlan plan = vlut_plan(p.rows, 3 * B, p.K, p.q, p.M, VLUT_METHOD_MFMA, p.prepared);
     // the plane sum goes into the plan's last kernel where that kernel holds
     // all three planes of an output: the rows kernel with one split and one
     // token tile, or the reduce of a split wide / deep kernel; a staged rows
@@ -1220,13 +1226,20 @@ hipError_t vlut_matmul(VlutMatmulArgs p, const VlutPlan& plan, hipStream_t s)
     p.pair_map = t->pair_map;
     p.pair_vals = t->pair_vals;
     if (p.prepared == VLUT_DECODED && plan.kernel != VK_MFMA_ROWS && plan.kernel != VK_MFMA_WIDE &&
-        plan.kernel != VK_MFMA_DEEP)
+        plan.kernel != VK_MFMA_DEEP && plan.kernel != VK_MFMA_GEMM)
         return hipErrorInvalidValue;
     if (p.prepared == VLUT_DECODED6) {
         // the rows and deep kernels read the 6-byte format
         const int off = decoded6_offset(*t, p.M);
-        if (off < 0 || (plan.kernel != VK_MFMA_ROWS && plan.kernel != VK_MFMA_DEEP)) return hipErrorInvalidValue;
+        if (off < 0 || (plan.kernel != VK_MFMA_ROWS && plan.kernel != VK_MFMA_DEEP && plan.kernel != VK_MFMA_GEMM))
+            return hipErrorInvalidValue;
         p.d6_bias = 2 * off;
+    }
+    if (plan.kernel == VK_MFMA_GEMM) {
+        // one pass over the whole K, no partials; decoded formats only
+        if (!p.swar_ok || (p.prepared != VLUT_DECODED && p.prepared != VLUT_DECODED6) || p.planes_b > 0)
+            return hipErrorInvalidValue;
+        return vlut_launch_gemm(p, plan.shape, s);
     }
     if (p.prepared == VLUT_PAIRS && plan.kernel != VK_LDS) return hipErrorInvalidValue;
     if (plan.kernel == VK_MFMA_WIDE || plan.kernel == VK_MFMA_DEEP || plan.kernel == VK_LDS) {

@@ -81,6 +81,9 @@ extern int g_vlut_swar;
 extern int g_vlut_splits;
 // 1 (default): batches above 32 tokens take the deep kernel, 0 the wide one
 extern int g_vlut_deep;
+// large batches of the decoded formats: 0 the deep kernel, 1 (default) the
+// GEMM kernel where the plan prefers it, 2 + s its shape s always
+extern int g_vlut_gemm;
 
 // Index of level word m of (row, k-block kb) in a weight of format fmt.
 // (VLUT_DECODED: index of the pair's first uint32; VLUT_DECODED6: of the
@@ -113,17 +116,22 @@ __host__ __device__ inline int64_t vlut_prepared_words(int64_t rows, int64_t kb,
 
 // Launch plan of a matmul: kernel and K splits (splits > 1 needs a
 // workspace of splits * B * rows floats and a reduce launch).
-enum VlutKernel { VK_LDS = 0, VK_MFMA_TILE = 1, VK_MFMA_ROWS = 2, VK_MFMA_WIDE = 3, VK_MFMA_DEEP = 4 };
+enum VlutKernel { VK_LDS = 0, VK_MFMA_TILE = 1, VK_MFMA_ROWS = 2, VK_MFMA_WIDE = 3, VK_MFMA_DEEP = 4,
+                  VK_MFMA_GEMM = 5 };
 struct VlutPlan {
     int kernel;
     int splits;
+    int shape;   // VK_MFMA_GEMM: its tile shape
 };
-VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method);
+// fmt: the weight's format, or -1 for the plan that serves every format (the
+// one workspaces are sized for)
+VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method, int fmt = -1);
 // Workspace floats a plan needs: the split-K partials ([B, rows, splits],
 // or [splits, B, rows] for the wide kernel), none when the rows or wide
 // kernel runs unsplit and writes the output itself.
 inline int64_t vlut_workspace_floats(const VlutPlan& plan, int64_t B, int64_t rows)
 {
+    if (plan.kernel == VK_MFMA_GEMM) return 0;
     if ((plan.kernel == VK_MFMA_ROWS || plan.kernel == VK_MFMA_WIDE || plan.kernel == VK_MFMA_DEEP ||
          plan.kernel == VK_LDS) &&
         plan.splits == 1)

@@ -212,5 +212,9 @@ hipError_t vlut_launch_rows(const VlutMatmulArgs& p, int splits, hipStream_t s);
 bool vlut_rows_staged(int64_t K, int splits);
 hipError_t vlut_launch_wide(const VlutMatmulArgs& p, int splits, hipStream_t s);
 hipError_t vlut_launch_deep(const VlutMatmulArgs& p, int splits, hipStream_t s);
+// The GEMM kernel of the decoded formats (vlut_gemm.hip) in tile shape
+// `shape`, and the shape the plan takes for these sizes (-1: the deep kernel).
+hipError_t vlut_launch_gemm(const VlutMatmulArgs& p, int shape, hipStream_t s);
+int vlut_gemm_shape(int64_t rows, int64_t B, int64_t K, int cus);
 
 }  // namespace coset

@@ -86,7 +86,8 @@ enum {
                                       beta = 2^k calls; the layer round trip's for stored or theta-derived betas at q = 4, 8, 16), 0 never */
     COSET_OPT_CODEC_DYNAMIC = 6,   /* fixed-format table kernel: 1 tiles from a counter run per launch (default), 0 grid stride */
     COSET_OPT_VLUT_DEEP = 7,       /* vLUT matmul above 32 tokens: 1 the 64-row deep kernel (default), 0 the 128-row wide one */
-    COSET_OPT_GEMM_TN_TILE = 8     /* coset_gemm_tn output tiles: 0 64 x 64 where they fit, else 96 x 96 (default); 64 or 96 only that size */
+    COSET_OPT_GEMM_TN_TILE = 8,    /* coset_gemm_tn output tiles: 0 64 x 64 where they fit, else 96 x 96 (default); 64 or 96 only that size */
+    COSET_OPT_VLUT_GEMM = 9        /* large vLUT batches of the decoded formats: 0 the deep kernel, 1 the GEMM kernel where the plan prefers it (default), 2..5 its tile shape 0..3 always */
 };
 
 int coset_abi_version(void);

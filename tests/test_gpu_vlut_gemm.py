@@ -1,0 +1,112 @@
+"""The GEMM kernel of the vLUT matmul (large batches of the decoded formats)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# exact products, fp32 sums of at most K terms in any order: well inside 2^-14
+# of the summands' magnitude (the bound of the other matrix-core kernels)
+RTOL = 2.0 ** -14
+
+
+def _weight(rows, K, q, M, seed):
+    import coset_amd as ca
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = 1.5 * torch.randn(rows * K // 8, 8, device="cuda", generator=g)
+    words = ca.hnlq_encode(x, q, M, 1.0).reshape(rows, K // 8, M)
+    W = ca.hnlq_decode(words.reshape(-1, M), q, M, None).reshape(rows, K).double()
+    return words, W, g
+
+
+@pytest.mark.parametrize("layout", ["decoded", "decoded6"])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [0, 1, 2, 3])
+@pytest.mark.parametrize("B,rows,K", [(1, 4, 8), (129, 40, 64), (257, 200, 72), (300, 259, 1064), (127, 193, 200)])
+def test_gemm_shapes_vs_dense(layout, dt, shape, B, rows, K):
+    """Every tile shape at the edges of its tiles (one token, one token past a
+    tile, ragged rows and k-blocks, K below one stage), with a dividing scale,
+    a bias and the LSQ epilogue, against the dense product in float64."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    words, W, g = _weight(rows, K, 4, 2, 7 * B + rows)
+    w = ca.vlut_prepare(words, 4, layout=layout)
+    a = torch.randn(B, K, device="cuda", generator=g).to(dt)
+    sc = torch.rand(rows, device="cuda", generator=g) + 0.5
+    bias = torch.randn(rows, device="cuda", generator=g)
+    try:
+        _lib.set_vlut_gemm(2 + shape)
+        y = ca.vlut_matmul(w, a, scale=sc)
+        yb = ca.vlut_matmul(w, a, scale=sc, scale_mode="div", bias=bias)
+        alpha = torch.tensor(3.0, device="cuda")
+        yl = ca.vlut_matmul(w, a, scale=sc, scale_mode="div", bias=bias, act_quant=(alpha, 127))
+    finally:
+        _lib.set_vlut_gemm(1)
+    ref, mag = a.double() @ W.t(), a.double().abs() @ W.t().abs()
+    assert ((y.double() - ref * sc).abs() <= RTOL * mag * sc).all()
+    assert ((yb.double() - (ref / sc + bias)).abs() <= RTOL * (mag / sc + bias.abs())).all()
+    m = ca.LSQActivation(bit_width=8, init_alpha=3.0).cuda()
+    with torch.no_grad():
+        assert torch.equal(yl, m(yb))          # the epilogue on the same sums
+
+
+def test_gemm_inf_activation_and_padding():
+    """An infinite activation reaches its own token only, and activations past
+    K are zero (0 x inf in the padding would make NaN)."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    words, W, g = _weight(72, 200, 4, 2, 3)    # 25 k-blocks: a ragged last stage
+    w = ca.vlut_prepare(words, 4, layout="decoded")
+    a = torch.randn(130, 200, device="cuda", generator=g).half()
+    a[7, 199] = float("inf")
+    try:
+        for shape in range(4):
+            _lib.set_vlut_gemm(2 + shape)
+            y = ca.vlut_matmul(w, a)
+            fin = torch.isfinite(y)
+            assert fin[:7].all() and fin[8:].all()
+            nz = W[:, 199] != 0
+            assert not fin[7][nz].any()
+    finally:
+        _lib.set_vlut_gemm(1)
+
+
+@pytest.mark.parametrize("B,rows,K", [(128, 768, 768), (1000, 1000, 1000), (700, 3072, 264)])
+def test_gemm_natural_plan_equals_deep(B, rows, K):
+    """Where the plan takes the GEMM kernel, its outputs agree with the deep
+    kernel's (the same exact products, summed in another order), for both
+    decoded formats bit for bit with each other, and fp32 activations run
+    through it as three planes."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    words, W, g = _weight(rows, K, 4, 2, B)
+    d8, d6 = (ca.vlut_prepare(words, 4, layout=lay) for lay in ("decoded", "decoded6"))
+    a = torch.randn(B, K, device="cuda", generator=g)
+    mag = a.double().abs() @ W.t().abs()
+    for act in (a.bfloat16(), a.half(), a):
+        y = ca.vlut_matmul(d8, act)
+        assert torch.equal(y, ca.vlut_matmul(d6, act))
+        try:
+            _lib.set_vlut_gemm(0)
+            y0 = ca.vlut_matmul(d8, act)
+        finally:
+            _lib.set_vlut_gemm(1)
+        assert ((y - y0).double().abs() <= 2.0 ** -16 * mag).all()
+
+
+def test_gemm_under_graph_capture():
+    """Replays equal the eager result (no workspace, no memset nodes)."""
+    import coset_amd as ca
+    words, W, g = _weight(768, 768, 4, 2, 5)
+    w = ca.vlut_prepare(words, 4, layout="decoded")
+    a = torch.randn(512, 768, device="cuda", generator=g).bfloat16()
+    want = ca.vlut_matmul(w, a)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ca.vlut_matmul(w, a)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
