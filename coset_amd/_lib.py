@@ -67,6 +67,7 @@ SIGNATURES = {
     "coset_colsum": [_vp, _int, _i64, _i64, _vp, _vp, _i64, _vp],
     "coset_gemm_tn_supported": [_i64, _i64, _i64],
     "coset_gemm_tn": [_vp, _i64, _vp, _i64, _vp, _i64, _int, _i64, _i64, _i64, _vp, _vp, _i64, _vp],
+    "coset_gemm_wgrad": [_vp, _i64, _vp, _i64, _vp, _i64, _int, _i64, _i64, _i64, _vp, _vp, _i64, _vp],
     "coset_vlut_matmul_noalloc": [_vp, _int, _vp, _int, _vp, _int, _i64, _i64, _i64, _int, _int, _int, _int, _vp,
                                   _vp],
     "coset_probe_empty": [_int, _int, _int, _vp, _vp],
@@ -84,6 +85,7 @@ SIZE_QUERIES = {
     "coset_lsq_workspace_floats": [_i64],
     "coset_colsum_workspace_floats": [_i64, _i64],
     "coset_gemm_tn_workspace_floats": [_i64, _i64, _i64],
+    "coset_gemm_wgrad_workspace_floats": [_i64, _i64, _i64],
     "coset_vlut_noalloc_scratch_floats": [],
 }
 
@@ -96,6 +98,7 @@ OPT_CODEC_DYNAMIC = 6
 OPT_VLUT_DEEP = 7
 OPT_GEMM_TN_TILE = 8
 OPT_VLUT_GEMM = 9
+OPT_GEMM_WGRAD = 10
 CODEC_AUTO, CODEC_GENERIC, CODEC_LUT = 0, 1, 2
 
 _lib = None
@@ -222,6 +225,12 @@ def set_vlut_gemm(mode: int) -> None:
     GEMM kernel where the plan prefers it (default), 2 + s its tile shape s
     (256 x 256, 256 x 192, 128 x 128 or 128 x 64 tokens x rows) always."""
     call("coset_set_option", OPT_VLUT_GEMM, int(mode))
+
+
+def set_gemm_wgrad_tile(mode: int) -> None:
+    """coset_gemm_wgrad's output tiles: 1 the plan's choice, 2 + i only shape
+    i (192 x 192, 128 x 128)."""
+    call("coset_set_option", OPT_GEMM_WGRAD, int(mode))
 
 
 def set_gemm_tn_tile(tile: int) -> None:

@@ -127,6 +127,10 @@ int coset_set_option(int key, int value)
         if (value < 0 || value > 1) return fail(COSET_EINVAL, "vLUT deep %d not in {0,1}", value);
         coset::g_vlut_deep = value;
         return COSET_OK;
+    case COSET_OPT_GEMM_WGRAD:
+        if (value < 1 || value > 3) return fail(COSET_EINVAL, "gemm_wgrad tile %d not in 1..3", value);
+        coset::g_gemm_wgrad = value;
+        return COSET_OK;
     case COSET_OPT_VLUT_GEMM:
         if (value < 0 || value > 5) return fail(COSET_EINVAL, "vLUT gemm %d not in 0..5", value);
         coset::g_vlut_gemm = value;
@@ -524,6 +528,37 @@ int coset_gemm_tn(const void* A, int64_t lda, const void* B, int64_t ldb, void* 
                                          ldc, out_dtype, M, N, K, plan, need > 0 ? workspace : nullptr, colsum,
                                          (hipStream_t)stream),
                      "gemm_tn launch");
+}
+
+int64_t coset_gemm_wgrad_workspace_floats(int64_t M, int64_t N, int64_t K)
+{
+    return coset::gemm_wgrad_workspace_floats(coset::gemm_wgrad_plan(M, N, K), M, N);
+}
+
+int coset_gemm_wgrad(const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int out_dtype,
+                     int64_t M, int64_t N, int64_t K, float* colsum, float* workspace, int64_t workspace_floats,
+                     void* stream)
+{
+    if (M < 0 || N < 0 || K < 0) return fail(COSET_EINVAL, "M, N, K must be >= 0");
+    if (out_dtype != COSET_F32 && out_dtype != COSET_BF16)
+        return fail(COSET_EUNSUPPORTED, "output dtype %d not supported (fp32, bf16)", out_dtype);
+    const coset::GemmWgradPlan plan = coset::gemm_wgrad_plan(M, N, K);
+    if (plan.shape < 0)
+        return fail(COSET_EUNSUPPORTED, "shape M=%lld N=%lld K=%lld not taken: M, N positive multiples of 8, K >= 1",
+                    (long long)M, (long long)N, (long long)K);
+    if (!A || !B || !C) return fail(COSET_EINVAL, "NULL buffer");
+    if (!aligned(A, 16) || !aligned(B, 16) || !aligned(C, 16)) return fail(COSET_EINVAL, "buffers must be 16-byte aligned");
+    if (lda < M || ldb < N || ldc < N || lda % 8 || ldb % 8 || ldc % 8)
+        return fail(COSET_EINVAL, "leading dimensions must cover the rows and be multiples of 8");
+    if (lda > (1 << 24) || ldb > (1 << 24)) return fail(COSET_EUNSUPPORTED, "leading dimensions above 2^24");
+    const int64_t need = coset::gemm_wgrad_workspace_floats(plan, M, N);
+    if (!workspace || workspace_floats < need)
+        return fail(COSET_EINVAL, "workspace too small: %lld floats needed", (long long)need);
+    if (!aligned(workspace, 16)) return fail(COSET_EINVAL, "workspace must be 16-byte aligned");
+    return check_hip(coset::gemm_wgrad_bf16(static_cast<const uint16_t*>(A), lda, static_cast<const uint16_t*>(B), ldb, C,
+                                            ldc, out_dtype == COSET_BF16, M, N, K, plan, workspace, colsum,
+                                            (hipStream_t)stream),
+                     "gemm_wgrad launch");
 }
 
 int coset_qat_stats_update(const float* W, int64_t tiles, int64_t tile_size, double momentum, float* sigma_ema,

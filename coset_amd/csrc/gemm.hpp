@@ -36,4 +36,20 @@ hipError_t gemm_tn_bf16(const uint16_t* A, int64_t lda, const uint16_t* B, int64
                         int out_dtype, int64_t M, int64_t N, int64_t K, const GemmTnPlan& plan, float* workspace,
                         float* colsum, hipStream_t s);
 
+// The same product for the shapes above: M, N multiples of 8, any K (ragged
+// too).  shape < 0: not taken; tiles_m x tiles_n output tiles, `splits` K
+// ranges of `stages` 64-token stages.
+struct GemmWgradPlan {
+    int shape;
+    int tiles_m, tiles_n;
+    int splits, stages;
+};
+GemmWgradPlan gemm_wgrad_plan(int64_t M, int64_t N, int64_t K);
+// 1 (default): the plan's choice of tile, 2 + i: only tile shape i
+extern int g_gemm_wgrad;
+int64_t gemm_wgrad_workspace_floats(const GemmWgradPlan& p, int64_t M, int64_t N);
+hipError_t gemm_wgrad_bf16(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, void* C, int64_t ldc,
+                           int out_bf16, int64_t M, int64_t N, int64_t K, const GemmWgradPlan& plan, float* workspace,
+                           float* colsum, hipStream_t s);
+
 }  // namespace coset

@@ -327,11 +327,10 @@ def colsum(g2: torch.Tensor) -> torch.Tensor:
     return out
 
 
-# 1: the weight gradient gy^T x runs on coset_gemm_tn where the shape and
-# dtypes allow it (coset_gemm_tn_supported, bf16), 0: always on torch.mm
-# (hipBLASLt)
+# 1: the weight gradient gy^T x runs on coset_gemm_tn or coset_gemm_wgrad where
+# the shape and dtypes allow it (bf16), 0: always on torch.mm (hipBLASLt)
 _GEMM_TN = [1]
-# 1: where coset_gemm_tn runs the weight gradient of a step, the bias
+# 1: where one of these kernels runs the weight gradient of a step, the bias
 # gradient's column sums come from the same launch (workgroups of their own
 # beside the product's tiles), so a step that forks its backward over two
 # streams (CapturedQATStep) leaves only dX on the second stream; 0: from
@@ -340,8 +339,8 @@ _FUSE_BIAS_GRAD = [1]
 
 
 def set_gemm_tn(enabled: bool) -> None:
-    """Route the layer's weight-gradient product to coset_gemm_tn (default)
-    or to torch.mm."""
+    """Route the layer's weight-gradient product to coset_gemm_tn and
+    coset_gemm_wgrad (default) or to torch.mm."""
     _GEMM_TN[0] = 1 if enabled else 0
 
 
@@ -383,16 +382,75 @@ def _gemm_tn_takes(g2: torch.Tensor, x2: torch.Tensor) -> bool:
             and bool(_lib.load().coset_gemm_tn_supported(g2.shape[1], x2.shape[1], g2.shape[0])))
 
 
+def gemm_wgrad(a: torch.Tensor, b: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
+               colsum: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """a^T b as gemm_tn, for M and N multiples of 8 and any K >= 1
+    (coset_gemm_wgrad).  None where the kernel does not take the shape, dtypes
+    or alignment (colsum then untouched)."""
+    if out_dtype is None:
+        out_dtype = a.dtype
+    if (a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16 or out_dtype not in (torch.bfloat16, torch.float32)
+            or a.dim() != 2 or b.dim() != 2 or a.shape[0] != b.shape[0] or not a.is_cuda or b.device != a.device):
+        return None
+    K, M = a.shape
+    N = b.shape[1]
+    if K < 1 or M < 8 or N < 8 or M % 8 or N % 8:
+        return None
+    if colsum is not None and (colsum.dtype != torch.float32 or colsum.numel() != M or not colsum.is_contiguous()):
+        raise ValueError("colsum must be a contiguous fp32 tensor of M elements")
+    a = a.contiguous()
+    b = b.contiguous()
+    if (a.data_ptr() | b.data_ptr()) % 16:
+        return None
+    lib = _lib.load()
+    out = torch.empty((M, N), dtype=out_dtype, device=a.device)
+    need = int(lib.coset_gemm_wgrad_workspace_floats(M, N, K))
+    ws = torch.empty(max(need, 4), dtype=torch.float32, device=a.device)
+    _lib.check("coset_gemm_wgrad", lib.coset_gemm_wgrad(a.data_ptr(), M, b.data_ptr(), N, out.data_ptr(), N,
+                                                       _lib.BF16 if out_dtype == torch.bfloat16 else _lib.F32, M, N,
+                                                       K, 0 if colsum is None else colsum.data_ptr(), ws.data_ptr(),
+                                                       need, _lib.stream_of(a)))
+    return out
+
+
+def _gemm_wgrad_takes(g2: torch.Tensor, x2: torch.Tensor, with_bias: bool) -> bool:
+    """Whether _weight_grad runs g2^T x2 on coset_gemm_wgrad, where
+    coset_gemm_tn does not take it.  Its column sums come free, while
+    coset_colsum costs 6-23 us beside the library's product: with a bias
+    gradient it was faster at every measured shape of up to 3072 x 3072
+    outputs (16384 tokens x 768 x 3072: 88 against 149 + 14 us; 1000 x 768 x
+    768: 15.4 against 13.0 + 6.5) but large outputs of few tokens (269 x 3072 x
+    2048: 21.6 against 13.7 + 6.6).  Without one the library is up to 25 %
+    faster below about 3000 tokens (755 x 1536 x 1024: 14.2 against 15.2),
+    slower above (3672 x 320 x 768: 29.6 against 18.0).  Larger outputs
+    (4096 x 4096 x 4096: 126 against 162) stay with the library."""
+    if not (_GEMM_TN[0] == 1 and g2.is_cuda and x2.device == g2.device and g2.dtype == x2.dtype == torch.bfloat16
+            and g2.dim() == 2 and x2.dim() == 2 and g2.shape[0] == x2.shape[0]):
+        return False
+    K, M = g2.shape
+    N = x2.shape[1]
+    if M < 8 or N < 8 or M % 8 or N % 8 or M * N > 3072 * 3072:
+        return False
+    if K < (512 if M * N > 1 << 22 else 1) or (not with_bias and K < 3000):
+        return False
+    # gemm_wgrad copies what is not contiguous; a contiguous operand has to be aligned
+    return not ((g2.is_contiguous() and g2.data_ptr() % 16) or (x2.is_contiguous() and x2.data_ptr() % 16))
+
+
 def _weight_grad(g2: torch.Tensor, x2: torch.Tensor, colsum: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """dW_q = g2^T x2: coset_gemm_tn where it applies (with colsum: also the
-    fp32 column sums of g2, the bias gradient, in the same pass), else
-    torch.mm (colsum must then be None)."""
+    """dW_q = g2^T x2: coset_gemm_tn or coset_gemm_wgrad where they apply (with
+    colsum: also the fp32 column sums of g2, the bias gradient, in the same
+    pass), else torch.mm (colsum must then be None)."""
     if _gemm_tn_takes(g2, x2):
         out = gemm_tn(g2, x2, colsum=colsum)
         if out is not None:
             return out
+    if _gemm_wgrad_takes(g2, x2, colsum is not None):
+        out = gemm_wgrad(g2, x2, colsum=colsum)
+        if out is not None:
+            return out
     if colsum is not None:
-        raise RuntimeError("column sums requested where coset_gemm_tn does not run")
+        raise RuntimeError("column sums requested where no weight-gradient kernel runs")
     return g2.t() @ x2
 
 
@@ -426,7 +484,7 @@ def _aux_stream(device: torch.device) -> "torch.cuda.Stream":
 
 class QATLinearFn(torch.autograd.Function):
     """y = x W_q^T + b, the layer's F.linear (coset/core/layers.py:478): the
-    weight gradient runs on coset_gemm_tn where it applies (bf16), with the
+    weight gradient runs on coset_gemm_tn or coset_gemm_wgrad where they apply (bf16), with the
     bias gradient's column sums in the same pass, the other products on
     hipBLASLt (torch.mm); elsewhere the bias gradient is the fp32 column sum
     of the output gradient (coset_colsum).  Either way a bf16 layer's fp32
@@ -462,7 +520,7 @@ class QATLinearFn(torch.autograd.Function):
             # branches of the graph.
             g2 = g2.contiguous()
             fuse = (_FUSE_BIAS_GRAD[0] == 1 and fast_db and g2.dtype == torch.bfloat16
-                    and _gemm_tn_takes(g2, x2))
+                    and (_gemm_tn_takes(g2, x2) or _gemm_wgrad_takes(g2, x2, True)))
             main = torch.cuda.current_stream(g2.device)
             aux = _aux_stream(g2.device)
             dx2 = torch.empty((g2.shape[0], Wq.shape[1]), dtype=g2.dtype, device=g2.device) if need_dx else None
@@ -486,7 +544,7 @@ class QATLinearFn(torch.autograd.Function):
         # one stream: the bias gradient in the weight-gradient kernel's pass
         # where that kernel runs (bf16), the column sums of gy with gy^T x
         if (_FUSE_BIAS_GRAD[0] == 1 and fast_db and need_dw and g2.dtype == torch.bfloat16 and g2.is_contiguous()
-                and _gemm_tn_takes(g2, x2)):
+                and (_gemm_tn_takes(g2, x2) or _gemm_wgrad_takes(g2, x2, True))):
             dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device)
             dW = _weight_grad(g2, x2, colsum=dbf)
             db = dbf.to(ctx.bias_dtype)

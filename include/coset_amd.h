@@ -87,7 +87,8 @@ enum {
     COSET_OPT_CODEC_DYNAMIC = 6,   /* fixed-format table kernel: 1 tiles from a counter run per launch (default), 0 grid stride */
     COSET_OPT_VLUT_DEEP = 7,       /* vLUT matmul above 32 tokens: 1 the 64-row deep kernel (default), 0 the 128-row wide one */
     COSET_OPT_GEMM_TN_TILE = 8,    /* coset_gemm_tn output tiles: 0 64 x 64 where they fit, else 96 x 96 (default); 64 or 96 only that size */
-    COSET_OPT_VLUT_GEMM = 9        /* large vLUT batches of the decoded formats: 0 the deep kernel, 1 the GEMM kernel where the plan prefers it (default), 2..5 its tile shape 0..3 always */
+    COSET_OPT_VLUT_GEMM = 9,       /* large vLUT batches of the decoded formats: 0 the deep kernel, 1 the GEMM kernel where the plan prefers it (default), 2..5 its tile shape 0..3 always */
+    COSET_OPT_GEMM_WGRAD = 10      /* coset_gemm_wgrad output tiles: 1 the plan's choice (default), 2, 3: 192 x 192 or 128 x 128 always */
 };
 
 int coset_abi_version(void);
@@ -241,6 +242,15 @@ int64_t coset_gemm_tn_workspace_floats(int64_t M, int64_t N, int64_t K);
 int coset_gemm_tn(const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int out_dtype,
                   int64_t M, int64_t N, int64_t K, float* colsum, float* workspace, int64_t workspace_floats,
                   void* stream);
+
+/* The same product for the shapes coset_gemm_tn does not take (many or ragged
+ * tokens, wide layers): M and N multiples of 8, any K >= 1, otherwise as
+ * coset_gemm_tn (leading dimensions up to 2^24); workspace: coset_gemm_wgrad_workspace_floats(M, N, K) floats,
+ * 16-byte aligned. */
+int64_t coset_gemm_wgrad_workspace_floats(int64_t M, int64_t N, int64_t K);
+int coset_gemm_wgrad(const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int out_dtype,
+                     int64_t M, int64_t N, int64_t K, float* colsum, float* workspace, int64_t workspace_floats,
+                     void* stream);
 
 /* The layer's periodic statistics update (HNLQLinearQAT._gather_stats,
  * coset/core/layers.py:366-379, run every stat_update_interval steps at
