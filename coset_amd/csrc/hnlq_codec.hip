@@ -498,14 +498,14 @@ __global__ void __launch_bounds__(256) hnlq_layer_rt_kernel(CodecArgs a)
 // Calls the layer round-trip kernel takes (its static_asserts, the domain of
 // its division and row index; it always tries the fast projection first);
 // g_codec_plain = 0 keeps them on the generic kernel.
-static bool layer_rt_supported(const CodecArgs& a, int mode)
+static bool layer_rt_supported(const CodecArgs& a, int mode, bool assume_tables = false)
 {
     // betas stored per row, or derived from theta per row of at least 64
     // blocks (fp32 weights: the layer quantizer's input)
     const bool betas = a.use_theta ? a.blocks_per_row >= 64 && a.x_dtype == DT_F32 : a.beta_row != nullptr;
     return g_codec_plain && a.fast_projection && mode == MODE_ROUNDTRIP && a.scale_mode == SCALE_LAYER && betas &&
            (a.q == 8 || a.q == 16 ||
-            (a.q == 4 && a.dec_map && ((uintptr_t)a.packed & 3u) == 0)) &&
+            (a.q == 4 && (a.dec_map || assume_tables) && ((uintptr_t)a.packed & 3u) == 0)) &&
            a.M >= 1 && a.M <= 4 &&
            !a.dither && !a.codes_f32 &&
            (a.x_dtype == DT_F32 || a.x_dtype == DT_BF16) && (a.out_dtype == DT_F32 || a.out_dtype == DT_BF16) &&
@@ -710,8 +710,13 @@ hipError_t launch_codec(const CodecArgs& args, int mode, hipStream_t s)
 {
     CodecArgs a = args;
     a.fast_projection = g_fast_projection;
-    bool lut = lut_path_supported(a, mode) &&
-               (g_codec_path == 2 || (g_codec_path == 0 && a.n >= kLutMinBlocks));
+    // the general table kernel leaves the layer quantizer with betas from
+    // theta to the layer round-trip kernel (3072 x 3072 to bf16: 33.5 -> 22.6 us)
+    const bool plain = lut_plain_supported(a, mode);
+    const int64_t from = !plain ? kLutMinBlocks : mode == MODE_ROUNDTRIP ? kLutMinBlocksPlainRt : kLutMinBlocksPlain;
+    const bool lut = lut_path_supported(a, mode) &&
+                     (g_codec_path == 2 ||
+                      (g_codec_path == 0 && a.n >= from && (plain || !layer_rt_supported(a, mode, true))));
     if (a.aux_out && a.aux_n > 0 && (lut || a.n == 0)) {
         // the table kernels take no side cast: it gets its own launch
         hipLaunchKernelGGL(aux_cast_kernel, dim3((unsigned)((a.aux_n + 255) / 256)), dim3(256), 0, s, a);

@@ -1,0 +1,118 @@
+"""The table codec's fixed-format kernels: bf16, per-row betas, dividing betas."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(fn):
+    """fn() on the fixed-format table kernel and on the generic kernel."""
+    from coset_amd import _lib
+    out = []
+    try:
+        for path, plain in ((2, True), (1, False)):
+            _lib.set_codec_path(path)
+            _lib.set_codec_plain(plain)
+            r = fn()
+            out.append(r if isinstance(r, tuple) else (r,))
+    finally:
+        _lib.set_codec_path(0)
+        _lib.set_codec_plain(True)
+    for a, b in zip(*out):
+        a, b = (v.view(torch.int16 if v.element_size() == 2 else torch.int32) for v in (a, b))
+        assert torch.equal(a, b)
+    return out[0]
+
+
+def _x(n, seed, zeros=True):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = 2 * torch.randn(n, 8, device="cuda", generator=g)
+    if zeros and n > 4:
+        x[1] = 0.0
+        x[2, ::2] = 0.0
+        x[3] = torch.tensor([0.5, -0.5, 1.5, -2.5, 1e-30, -0.0, 3e-39, 2.0], device="cuda")
+    return x
+
+
+@pytest.mark.parametrize("q,M", [(4, 1), (4, 2), (2, 3), (2, 4)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,per_row", [(1, 1), (3, 21), (129, 512), (40, 65)])
+def test_per_row_betas(q, M, dt, rows, per_row):
+    """Encode, decode and round trip with stored per-row betas (ordinary, zero,
+    negative, tiny, huge, non-finite) and a clip, against the generic kernel
+    bit for bit in both output types."""
+    import coset_amd as ca
+    n = rows * per_row
+    x = _x(n, n).to(dt)
+    beta = 0.5 + torch.rand(rows, device="cuda")
+    odd = torch.tensor([1e-30, 1e30, -0.7, float("inf"), 0.0, 3e38, 1e-44, float("nan")], device="cuda")
+    k = min(rows, len(odd))
+    if rows > 1:
+        beta[:k] = odd[:k]
+    kw = dict(beta_row=beta, blocks_per_row=per_row)
+    words = _both(lambda: ca.hnlq_encode(x, q, M, **kw))[0]
+    for od in (torch.float32, torch.bfloat16):
+        for clip in (float("inf"), 1.25):
+            _both(lambda: ca.hnlq_decode(words, q, M, clip=clip, out_dtype=od, **kw))
+            _both(lambda: ca.hnlq_roundtrip(x, q, M, clip=clip, out_dtype=od, **kw))
+        _both(lambda: ca.hnlq_decode(words, q, M, clip=0.0, out_dtype=od, **kw))
+
+
+@pytest.mark.parametrize("q,M", [(4, 2), (4, 3), (2, 4)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("beta", [None, 0.25, 0.3, 0.02, 7.1, 1e-7, 1e7])
+def test_codec_betas_and_dtypes(q, M, dt, beta):
+    """No scale, powers of two, and betas that divide (one inside, two outside
+    the fixed-format kernel's range), values from denormal to 2^21 and beyond,
+    infinities and NaN: bit for bit the generic kernel's."""
+    import coset_amd as ca
+    n = 3000
+    x = _x(n, 5)
+    x *= torch.exp2(torch.randint(-30, 20, (n, 1), device="cuda").float())
+    x[7, 0], x[8, 1], x[9, 2] = float("inf"), float("nan"), 1e38
+    x = x.to(dt)
+    words = _both(lambda: ca.hnlq_encode(x, q, M, beta))[0]
+    _both(lambda: ca.hnlq_roundtrip(x, q, M, beta))
+    if dt == torch.float32:
+        _both(lambda: ca.hnlq_encode(x, q, M, beta, return_codes=True))
+    for od in (torch.float32, torch.bfloat16):
+        _both(lambda: ca.hnlq_decode(words, q, M, beta, out_dtype=od))
+
+
+def test_dividing_beta_matches_oracle():
+    """x / beta through the shared reciprocal against the oracle's division."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    x = 3 * torch.randn(20000, 8, device="cuda")
+    try:
+        _lib.set_codec_path(2)
+        for beta in (0.3, 0.02, 1.7, 123.4):
+            b = float(np.float32(beta))
+            words = ca.hnlq_encode(x * beta, 4, 2, b)
+            codes = O.e8_encode((x * beta).cpu().numpy(), 4, 2, b)
+            assert np.array_equal(words.cpu().numpy().astype(np.uint32), O.pack_words(codes, 4))
+    finally:
+        _lib.set_codec_path(0)
+
+
+@pytest.mark.parametrize("n", [(1 << 18) - 1, 1 << 18, (1 << 19) + 77, (6 << 20) - 1, (6 << 20) + 1])
+def test_sizes_around_the_dispatch_lines(n):
+    """The natural route below and above each line (table kernel, counter
+    tiles) equals the generic kernel."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    x = _x(n, 9)
+    got = ca.hnlq_roundtrip(x, 4, 2, None)
+    words = ca.hnlq_encode(x, 4, 2, None)
+    dec = ca.hnlq_decode(words, 4, 2, None)
+    try:
+        _lib.set_codec_path(1)
+        want = ca.hnlq_roundtrip(x, 4, 2, None)
+    finally:
+        _lib.set_codec_path(0)
+    s = torch.int16
+    assert torch.equal(got[0].view(s), want[0].view(s)) and torch.equal(words.view(s), want[0].view(s))
+    assert torch.equal(got[1], want[1]) and torch.equal(dec, want[1])
