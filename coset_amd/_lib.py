@@ -135,8 +135,16 @@ def load():
     return lib
 
 
+_fns = {}
+
+
 def call(name: str, *args) -> None:
-    check(name, getattr(load(), name)(*args))
+    f = _fns.get(name)
+    if f is None:
+        f = _fns[name] = getattr(load(), name)
+    rc = f(*args)
+    if rc != OK:
+        check(name, rc)
 
 
 def word_bytes(q: int) -> int:

@@ -91,6 +91,8 @@ def default_device(device=None) -> torch.device:
 
 def on_gpu(t: torch.Tensor) -> torch.Tensor:
     """The tensor on the current GPU (a copy when it lives on the host)."""
+    if t.is_cuda and t.get_device() in _lib._inited:   # every call of a running program
+        return t
     dev = _lib.require_gpu()
     if t.device.type != "cuda":
         t = t.to(dev)

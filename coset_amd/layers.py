@@ -199,12 +199,29 @@ def qat_fwd_theta(Wc, theta, sigma, xmax, step_count, bounds, q, M, clip, blocks
             raise ValueError(f"bias must hold {rows} values")
         b_out = torch.empty(rows, dtype=out_dtype, device=dev)
     delta0, eta, ginv, m_bounds = bounds
-    _lib.check("coset_e8_qat_fwd_theta", _lib.fn("coset_e8_qat_fwd_theta")(
-        Wc.data_ptr(), rows, cols, blocks_per_tile, th.data_ptr(), sigma.contiguous().data_ptr(),
-        xmax.contiguous().data_ptr(), delta0, eta, ginv, m_bounds, clip, q, M, Wq.data_ptr(),
-        _lib.dtype_code(out_dtype), packed.data_ptr(), beta.data_ptr(), dbdt.data_ptr(),
-        _lib.ptr(step_count), _lib.ptr(b_in), _lib.ptr(b_out), _lib.stream_of(Wc)))
+    _lib.call("coset_e8_qat_fwd_theta",
+              Wc.data_ptr(), rows, cols, blocks_per_tile, th.data_ptr(), sigma.contiguous().data_ptr(),
+              xmax.contiguous().data_ptr(), delta0, eta, ginv, m_bounds, clip, q, M, Wq.data_ptr(),
+              _lib.dtype_code(out_dtype), packed.data_ptr(), beta.data_ptr(), dbdt.data_ptr(),
+              _lib.ptr(step_count), _lib.ptr(b_in), _lib.ptr(b_out), _lib.stream_of(Wc))
     return Wq, packed, beta, dbdt, b_out
+
+
+def qat_bwd_theta(g, Wc, packed, beta, dbdt, q, M, clip, blocks_per_tile, theta_shape):
+    """One coset_e8_qat_bwd_theta call: (dW, dtheta) from the gradient of W_q
+    and what qat_fwd_theta returned."""
+    if g.dtype not in (torch.float32, torch.bfloat16):
+        g = g.float()
+    g = g.contiguous()
+    rows, cols = Wc.shape
+    dW = torch.empty_like(Wc)
+    dbeta = torch.empty_like(beta)
+    dtheta = torch.empty_like(beta)
+    _lib.call("coset_e8_qat_bwd_theta",
+              g.data_ptr(), _lib.dtype_code(g.dtype), Wc.data_ptr(), packed.data_ptr(), beta.data_ptr(),
+              dbdt.data_ptr(), rows, cols, blocks_per_tile, clip, q, M, dW.data_ptr(), dbeta.data_ptr(),
+              dtheta.data_ptr(), _lib.stream_of(Wc))
+    return dW, dtheta.view(theta_shape)
 
 
 class E8ThetaWeightQuant(torch.autograd.Function):
@@ -236,20 +253,8 @@ class E8ThetaWeightQuant(torch.autograd.Function):
     def backward(ctx, g, g_bias=None):
         if g is None:
             return (None,) * 12
-        Wc, packed, beta, dbdt = ctx.saved_tensors
-        q, M, clip, bpt, theta_shape = ctx.cfg
-        if g.dtype not in (torch.float32, torch.bfloat16):
-            g = g.float()
-        g = g.contiguous()
-        rows, cols = Wc.shape
-        dW = torch.empty_like(Wc)
-        dbeta = torch.empty_like(beta)
-        dtheta = torch.empty_like(beta)
-        _lib.check("coset_e8_qat_bwd_theta", _lib.fn("coset_e8_qat_bwd_theta")(
-            g.data_ptr(), _lib.dtype_code(g.dtype), Wc.data_ptr(), packed.data_ptr(), beta.data_ptr(),
-            dbdt.data_ptr(), rows, cols, bpt, clip, q, M, dW.data_ptr(), dbeta.data_ptr(), dtheta.data_ptr(),
-            _lib.stream_of(Wc)))
-        return dW, dtheta.view(theta_shape), None, None, None, None, None, None, None, None, None, None
+        dW, dtheta = qat_bwd_theta(g, *ctx.saved_tensors, *ctx.cfg)
+        return dW, dtheta, None, None, None, None, None, None, None, None, None, None
 
 
 def d4_qat_fwd_theta(Wc, theta, sigma, xmax, step_count, bounds, q, clip, blocks_per_tile, out_dtype):
@@ -482,6 +487,69 @@ def _aux_stream(device: torch.device) -> "torch.cuda.Stream":
     return s
 
 
+def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: bool):
+    """(dx, dW_q, db) of y = x W_q^T + b, None where not needed; bias_dtype is
+    None without a bias."""
+    need_db = need_db and bias_dtype is not None
+    g2 = gy.reshape(-1, gy.shape[-1])
+    dx = dW = db = None
+    fast_db = (need_db and g2.shape[1] % 8 == 0
+               and g2.dtype in (torch.float32, torch.bfloat16, torch.float16))
+    overlap = g2.is_cuda and (_OVERLAP_BACKWARD[0] > 0 or torch.cuda.is_current_stream_capturing())
+    x2 = x.reshape(-1, x.shape[-1])
+    if overlap and need_dw and (need_dx or fast_db) and g2.dtype == Wq.dtype == x.dtype:
+        # dX (and the bias gradient where coset_gemm_tn does not take it)
+        # on a second stream while dW runs on this one: the dW product
+        # alone leaves CUs idle at these shapes (one 64 x 64 or 128 x 128
+        # tile per CU or fewer).  Outputs are allocated here, on the
+        # current stream, before the fork; the join comes before they are
+        # returned.  Under graph capture the two streams become two
+        # branches of the graph.
+        g2 = g2.contiguous()
+        fuse = (_FUSE_BIAS_GRAD[0] == 1 and fast_db and g2.dtype == torch.bfloat16
+                and (_gemm_tn_takes(g2, x2) or _gemm_wgrad_takes(g2, x2, True)))
+        main = torch.cuda.current_stream(g2.device)
+        aux = _aux_stream(g2.device)
+        dx2 = torch.empty((g2.shape[0], Wq.shape[1]), dtype=g2.dtype, device=g2.device) if need_dx else None
+        cs = _colsum_buffers(g2) if fast_db and not fuse else None
+        dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device) if fuse else None
+        aux.wait_stream(main)
+        with torch.cuda.stream(aux):
+            if need_dx:
+                torch.mm(g2, Wq, out=dx2)
+            if cs is not None:
+                _colsum_into(g2, *cs)
+        dW = _weight_grad(g2, x2, colsum=dbf)
+        main.wait_stream(aux)
+        if need_dx:
+            dx = dx2.reshape(x.shape)
+        if fast_db:
+            db = (dbf if fuse else cs[0]).to(bias_dtype)
+        elif need_db:
+            db = g2.float().sum(0).to(bias_dtype)
+        return dx, dW, db
+    # one stream: the bias gradient in the weight-gradient kernel's pass
+    # where that kernel runs (bf16), the column sums of gy with gy^T x
+    if (_FUSE_BIAS_GRAD[0] == 1 and fast_db and need_dw and g2.dtype == torch.bfloat16 and g2.is_contiguous()
+            and (_gemm_tn_takes(g2, x2) or _gemm_wgrad_takes(g2, x2, True))):
+        dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device)
+        dW = _weight_grad(g2, x2, colsum=dbf)
+        db = dbf.to(bias_dtype)
+        if need_dx:
+            dx = (g2 @ Wq).reshape(x.shape)
+        return dx, dW, db
+    if need_dx:
+        dx = (g2 @ Wq).reshape(x.shape)
+    if need_dw:
+        dW = _weight_grad(g2, x2)
+    if need_db:
+        if g2.shape[1] % 8 == 0 and g2.dtype in (torch.float32, torch.bfloat16, torch.float16):
+            db = colsum(g2).to(bias_dtype)
+        else:
+            db = g2.float().sum(0).to(bias_dtype)
+    return dx, dW, db
+
+
 class QATLinearFn(torch.autograd.Function):
     """y = x W_q^T + b, the layer's F.linear (coset/core/layers.py:478): the
     weight gradient runs on coset_gemm_tn or coset_gemm_wgrad where they apply (bf16), with the
@@ -503,64 +571,41 @@ class QATLinearFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gy):
         x, Wq = ctx.saved_tensors
-        g2 = gy.reshape(-1, gy.shape[-1])
-        dx = dW = db = None
-        need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        fast_db = (ctx.bias_dtype is not None and ctx.needs_input_grad[2] and g2.shape[1] % 8 == 0
-                   and g2.dtype in (torch.float32, torch.bfloat16, torch.float16))
-        overlap = g2.is_cuda and (_OVERLAP_BACKWARD[0] > 0 or torch.cuda.is_current_stream_capturing())
-        x2 = x.reshape(-1, x.shape[-1])
-        if overlap and need_dw and (need_dx or fast_db) and g2.dtype == Wq.dtype == x.dtype:
-            # dX (and the bias gradient where coset_gemm_tn does not take it)
-            # on a second stream while dW runs on this one: the dW product
-            # alone leaves CUs idle at these shapes (one 64 x 64 or 128 x 128
-            # tile per CU or fewer).  Outputs are allocated here, on the
-            # current stream, before the fork; the join comes before they are
-            # returned.  Under graph capture the two streams become two
-            # branches of the graph.
-            g2 = g2.contiguous()
-            fuse = (_FUSE_BIAS_GRAD[0] == 1 and fast_db and g2.dtype == torch.bfloat16
-                    and (_gemm_tn_takes(g2, x2) or _gemm_wgrad_takes(g2, x2, True)))
-            main = torch.cuda.current_stream(g2.device)
-            aux = _aux_stream(g2.device)
-            dx2 = torch.empty((g2.shape[0], Wq.shape[1]), dtype=g2.dtype, device=g2.device) if need_dx else None
-            cs = _colsum_buffers(g2) if fast_db and not fuse else None
-            dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device) if fuse else None
-            aux.wait_stream(main)
-            with torch.cuda.stream(aux):
-                if need_dx:
-                    torch.mm(g2, Wq, out=dx2)
-                if cs is not None:
-                    _colsum_into(g2, *cs)
-            dW = _weight_grad(g2, x2, colsum=dbf)
-            main.wait_stream(aux)
-            if need_dx:
-                dx = dx2.reshape(x.shape)
-            if fast_db:
-                db = (dbf if fuse else cs[0]).to(ctx.bias_dtype)
-            elif ctx.bias_dtype is not None and ctx.needs_input_grad[2]:
-                db = g2.float().sum(0).to(ctx.bias_dtype)
-            return dx, dW, db, None
-        # one stream: the bias gradient in the weight-gradient kernel's pass
-        # where that kernel runs (bf16), the column sums of gy with gy^T x
-        if (_FUSE_BIAS_GRAD[0] == 1 and fast_db and need_dw and g2.dtype == torch.bfloat16 and g2.is_contiguous()
-                and (_gemm_tn_takes(g2, x2) or _gemm_wgrad_takes(g2, x2, True))):
-            dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device)
-            dW = _weight_grad(g2, x2, colsum=dbf)
-            db = dbf.to(ctx.bias_dtype)
-            if need_dx:
-                dx = (g2 @ Wq).reshape(x.shape)
-            return dx, dW, db, None
-        if ctx.needs_input_grad[0]:
-            dx = (g2 @ Wq).reshape(x.shape)
-        if ctx.needs_input_grad[1]:
-            dW = _weight_grad(g2, x.reshape(-1, x.shape[-1]))
-        if ctx.bias_dtype is not None and ctx.needs_input_grad[2]:
-            if g2.shape[1] % 8 == 0 and g2.dtype in (torch.float32, torch.bfloat16, torch.float16):
-                db = colsum(g2).to(ctx.bias_dtype)
-            else:
-                db = g2.float().sum(0).to(ctx.bias_dtype)
-        return dx, dW, db, None
+        need = ctx.needs_input_grad
+        return (*linear_grads(gy, x, Wq, ctx.bias_dtype, need[0], need[1], need[2]), None)
+
+
+class QATLayerFn(torch.autograd.Function):
+    """The fused layer as one autograd node: W_q as E8ThetaWeightQuant makes it,
+    y = x W_q^T + b as QATLinearFn does, and both backwards in turn.  cfg:
+    (bounds, q, M, clip, blocks_per_tile).  Half the nodes of the two functions
+    one after the other, whose Python and engine overhead an eager step of a
+    small batch waits for."""
+
+    @staticmethod
+    def forward(ctx, x, W, theta, bias, sigma, xmax, step_count, cfg):
+        bounds, q, M, clip, bpt = cfg
+        Wc = W.detach().contiguous()
+        # a bf16 product takes the bias in bf16, written in the launch that writes W_q
+        cast = bias is not None and x.dtype == torch.bfloat16
+        Wq, packed, beta, dbdt, b_cast = qat_fwd_theta(Wc, theta.detach(), sigma, xmax, step_count, bounds, q, M, clip,
+                                                       bpt, x.dtype, bias if cast else None)
+        ctx.save_for_backward(x, Wq, Wc, packed, beta, dbdt)
+        ctx.cfg = (q, M, clip, bpt, theta.shape)
+        ctx.bias_dtype = None if bias is None else bias.dtype
+        if bias is not None and b_cast is None:
+            b_cast = bias.to(x.dtype)
+        return F.linear(x, Wq, b_cast)
+
+    @staticmethod
+    def backward(ctx, gy):
+        x, Wq, Wc, packed, beta, dbdt = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        dx, dWq, db = linear_grads(gy, x, Wq, ctx.bias_dtype, need[0], need[1] or need[2], need[3])
+        dW = dtheta = None
+        if dWq is not None:
+            dW, dtheta = qat_bwd_theta(dWq, Wc, packed, beta, dbdt, *ctx.cfg)
+        return dx, dW if need[1] else None, dtheta if need[2] else None, db, None, None, None, None
 
 
 class HNLQLinearQAT(nn.Module):
@@ -813,27 +858,34 @@ class HNLQLinearQAT(nn.Module):
         """Whether forward() runs as one fused launch (coset_e8_qat_head_fwd):
         a no-grad forward of at most 64 fp32 tokens through the fused E8
         quantizer with row tiling and q = 2, 4."""
-        if not (_HEAD_FWD[0] == 1 and x.is_cuda and x.dtype == torch.float32 and self.quantization_enabled
-                and self._fused() and self.tiling == "row" and self.q in (2, 4) and not self.enable_diagnostics
-                and x.shape[-1] == self.in_features and self.in_features <= 8192 and x.numel() > 0
-                and x.numel() // self.in_features <= 64):
+        cols = self.in_features
+        if not (x.dtype == torch.float32 and x.is_cuda and _HEAD_FWD[0] == 1 and 0 < x.numel() <= 64 * cols
+                and x.shape[-1] == cols and cols <= 8192 and self.quantization_enabled and self.tiling == "row"
+                and self.q in (2, 4) and not self.enable_diagnostics and self._fused()):
             return False
+        if not torch.is_grad_enabled():
+            return True
         params = (self.weight, self.theta_beta) + ((self.bias,) if self.bias is not None else ())
-        return not torch.is_grad_enabled() or not (x.requires_grad or any(p.requires_grad for p in params))
+        return not (x.requires_grad or any(p.requires_grad for p in params))
 
     def _head_forward(self, x):
         """y = x W_q^T + bias with W_q quantized in the same launch."""
         self._advance_step(device_increment=False)   # the kernel increments step_count
-        x2 = x.reshape(-1, self.in_features).contiguous()
-        y = torch.empty((x2.shape[0], self.out_features), dtype=torch.float32, device=x.device)
-        W = self.weight.detach().contiguous()
-        _lib.call("coset_e8_qat_head_fwd", W.data_ptr(), self.out_features, self.in_features,
-                  self.theta_beta.detach().contiguous().data_ptr(), self.sigma_ema.data_ptr(),
+        cols, rows = self.in_features, self.out_features
+        x2 = x if x.dim() == 2 and x.is_contiguous() else x.reshape(-1, cols).contiguous()
+        y = torch.empty((x2.shape[0], rows), dtype=torch.float32, device=x.device)
+        W, theta, bias = self.weight, self.theta_beta, self.bias
+        if not W.is_contiguous():
+            W = W.detach().contiguous()
+        if not theta.is_contiguous():
+            theta = theta.detach().contiguous()
+        _lib.call("coset_e8_qat_head_fwd", W.data_ptr(), rows, cols, theta.data_ptr(), self.sigma_ema.data_ptr(),
                   self.xmax_ema.data_ptr(), float(self.Delta0), float(self.eta), self._ginv_f, int(self.M),
                   float(self.weight_clip_value), int(self.q), x2.data_ptr(), x2.shape[0],
-                  None if self.bias is None else self.bias.detach().data_ptr(), y.data_ptr(),
+                  None if bias is None else bias.data_ptr(), y.data_ptr(),
                   self.step_count.data_ptr(), _lib.stream_of(x2))
-        y = y.reshape(*x.shape[:-1], self.out_features)
+        if x.dim() != 2:
+            y = y.reshape(*x.shape[:-1], rows)
         if self.quantize_activations and self.actq is not None:
             y = self.actq(y)
         return y
@@ -844,6 +896,15 @@ class HNLQLinearQAT(nn.Module):
         of up to 64 fp32 tokens run as one launch (quantizer and product)."""
         if self._head_takes(x):
             return self._head_forward(x)
+        if (x.is_cuda and self.quantization_enabled and not self.enable_diagnostics and self._fused()
+                and x.dtype in (torch.float32, torch.bfloat16)):
+            self._advance_step(device_increment=False)   # the kernel increments step_count
+            bpt = self.blocks_per_row if self.tiling == "row" else 1
+            x = QATLayerFn.apply(x, self.weight, self.theta_beta, self.bias, self.sigma_ema, self.xmax_ema,
+                                 self.step_count,
+                                 ((float(self.Delta0), float(self.eta), self._ginv_f, int(self.M)), int(self.q), 2,
+                                  float(self.weight_clip_value), int(bpt)))
+            return self.actq(x) if self.quantize_activations and self.actq is not None else x
         wdt = x.dtype if x.dtype in (torch.bfloat16, torch.float16) else torch.float32
         if wdt == torch.float16:
             wdt = torch.float32
