@@ -623,8 +623,20 @@ __global__ void __launch_bounds__(256) vlut_reduce_kernel(const float* partial, 
     out[i] = vlut_epilogue(acc * mult * sc, o, bias, lsq_alpha, lsq_qmax);
 }
 
+// acc + low <- acc + low + w with the rounding error of acc + w kept in low
+// (Knuth's two-sum); a sum that is not finite leaves low not finite, and the
+// callers then drop it
+__device__ __forceinline__ void two_sum(float& acc, float& low, float w)
+{
+    const float t = __fadd_rn(acc, w), b = __fsub_rn(t, acc);
+    low = __fadd_rn(low, __fadd_rn(__fsub_rn(acc, __fsub_rn(t, b)), __fsub_rn(w, b)));
+    acc = t;
+}
+
 // Same for partials stored split-major, [splits][B][rows] (the wide kernel);
 // the splits are summed in order.
+// COMP: compensated, for the GEMM kernel's many splits (below).
+template <bool COMP>
 __global__ void __launch_bounds__(256) vlut_reduce_sm_kernel(const float* partial, int splits, int64_t B,
                                                             int64_t rows, const float* scale, int scale_mode,
                                                             float mult, const float* bias, const float* lsq_alpha,
@@ -634,8 +646,14 @@ __global__ void __launch_bounds__(256) vlut_reduce_sm_kernel(const float* partia
     if (i >= B * rows) return;
     int64_t o = i % rows;
     const int64_t n = B * rows;
-    float acc = 0.f;
-    for (int s = 0; s < splits; ++s) acc += partial[s * n + i];
+    float acc = 0.f, low = 0.f;
+    for (int s = 0; s < splits; ++s) {
+        if constexpr (COMP)
+            two_sum(acc, low, partial[s * n + i]);
+        else
+            acc += partial[s * n + i];
+    }
+    if (COMP && low - low == 0.f) acc = __fadd_rn(acc, low);
     float sc = scale ? (scale_mode == 0 ? scale[o] : 1.f / scale[o]) : 1.f;
     out[i] = vlut_epilogue(acc * mult * sc, o, bias, lsq_alpha, lsq_qmax);
 }
@@ -676,6 +694,10 @@ __global__ void __launch_bounds__(256) vlut_reduce_sm4_kernel(const float* parti
 // thread: x runs on the XCD whose workgroups wrote that row group's
 // partials (both grids deal workgroups to the 8 XCDs by x mod 8 when there
 // are a multiple of 8 row groups), so its reads hit that XCD's L2.
+// COMP (the GEMM kernel's partials, up to 64 splits at few tokens): the sums
+// compensated, so many splits cost no precision (fp32, 48 tokens of 768 x 3072:
+// 8.6e-8 against 64 bits added in turn, the deep kernel's four splits 6.2e-8).
+template <bool COMP>
 __global__ void __launch_bounds__(256) vlut_reduce_rg4_kernel(const float* partial, int splits, int64_t B,
                                                              int64_t rows, const float* scale, int scale_mode,
                                                              float mult, const float* bias, const float* lsq_alpha,
@@ -687,13 +709,24 @@ __global__ void __launch_bounds__(256) vlut_reduce_rg4_kernel(const float* parti
     if (qd >= rq || tok >= B) return;
     const float4* p4 = reinterpret_cast<const float4*>(partial);
     const int64_t i4 = tok * rq + qd, o0 = 4 * qd;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    float acc[4] = {0.f, 0.f, 0.f, 0.f}, low[4] = {0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < splits; ++s) {
         const float4 v = p4[s * n4 + i4];
-        acc[0] += v.x;
-        acc[1] += v.y;
-        acc[2] += v.z;
-        acc[3] += v.w;
+        if constexpr (COMP) {
+            const float w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) two_sum(acc[j], low[j], w[j]);
+        } else {
+            acc[0] += v.x;
+            acc[1] += v.y;
+            acc[2] += v.z;
+            acc[3] += v.w;
+        }
+    }
+    if constexpr (COMP) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (low[j] - low[j] == 0.f) acc[j] = __fadd_rn(acc[j], low[j]);
     }
     float r[4];
 #pragma unroll
@@ -945,8 +978,9 @@ VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method,
     const bool swar = g_vlut_swar && ((q == 2 && M <= 4) || (q == 4 && M <= 2));
     if (swar && g_vlut_deep && g_vlut_gemm && g_vlut_splits == 0 &&
         (fmt == VLUT_DECODED || fmt == VLUT_DECODED6)) {
-        const int shape = g_vlut_gemm >= 2 ? g_vlut_gemm - 2 : vlut_gemm_shape(rows, B, K, device_cu_count());
-        if (shape >= 0) return {VK_MFMA_GEMM, 1, shape};
+        if (g_vlut_gemm >= 2) return {VK_MFMA_GEMM, 1, g_vlut_gemm - 2};
+        const VlutPlan g = vlut_gemm_plan(rows, B, K, device_cu_count());
+        if (g.kernel == VK_MFMA_GEMM) return g;
     }
     if (swar && B > 32 && g_vlut_deep) {
         // 64-row, 64-token workgroups, at most 32 k-quads each: enough K
@@ -1153,6 +1187,9 @@ __global__ void __launch_bounds__(256) vlut_split_sum_kernel(const float* __rest
 
 namespace {
 
+// Tokens from which fp32 activations take the GEMM kernel's own split
+constexpr int64_t kGemm32Tokens = 48;
+
 constexpr int64_t align64(int64_t n) { return (n + 63) / 64 * 64; }
 
 }  // namespace
@@ -1181,6 +1218,17 @@ hipError_t vlut_matmul_split(VlutMatmulArgs p, float* workspace, hipStream_t s)
     // kernel also splits the fp32 activations itself
     const bool v4 = p.rows % 4 == 0 && ((uintptr_t)p.out % 16) == 0 && ((uintptr_t)inner % 16) == 0;
     const bool rows1 = plan.kernel == VK_MFMA_ROWS && plan.splits == 1;
+    if ((p.prepared == VLUT_DECODED || p.prepared == VLUT_DECODED6) && g_vlut_deep && g_vlut_gemm && g_vlut_swar &&
+        g_vlut_splits == 0 && B >= kGemm32Tokens) {
+        // the GEMM kernel splits the fp32 activations itself, in one launch
+        // and a reduce; its partials fit the workspace's splits
+        const int64_t room = vlut_split_workspace_floats(B, p.rows, p.K, p.q, p.M) / std::max<int64_t>(1, B * p.rows);
+        VlutMatmulArgs f = p;
+        f.partial = workspace;
+        const VlutPlan plan32 = g_vlut_gemm >= 2 ? VlutPlan{VK_MFMA_GEMM, 1, std::min(g_vlut_gemm - 2, 2)}
+                                                 : vlut_gemm32_plan(p.rows, B, p.K, device_cu_count(), room);
+        return vlut_matmul(f, plan32, s);
+    }
     if (rows1 && 3 * B <= 15 && vlut_rows_staged(p.K, 1)) {
         q.planes_b = B;
         q.act_planes = 1;   // q.act stays the fp32 activations
@@ -1235,15 +1283,15 @@ hipError_t vlut_matmul(VlutMatmulArgs p, const VlutPlan& plan, hipStream_t s)
             return hipErrorInvalidValue;
         p.d6_bias = 2 * off;
     }
-    if (plan.kernel == VK_MFMA_GEMM) {
-        // one pass over the whole K, no partials; decoded formats only
-        if (!p.swar_ok || (p.prepared != VLUT_DECODED && p.prepared != VLUT_DECODED6) || p.planes_b > 0)
-            return hipErrorInvalidValue;
-        return vlut_launch_gemm(p, plan.shape, s);
-    }
+    if (plan.kernel == VK_MFMA_GEMM &&
+        (!p.swar_ok || (p.prepared != VLUT_DECODED && p.prepared != VLUT_DECODED6) || p.planes_b > 0))
+        return hipErrorInvalidValue;   // decoded formats only
     if (p.prepared == VLUT_PAIRS && plan.kernel != VK_LDS) return hipErrorInvalidValue;
-    if (plan.kernel == VK_MFMA_WIDE || plan.kernel == VK_MFMA_DEEP || plan.kernel == VK_LDS) {
-        if (plan.kernel == VK_LDS) {
+    if (plan.kernel == VK_MFMA_WIDE || plan.kernel == VK_MFMA_DEEP || plan.kernel == VK_MFMA_GEMM ||
+        plan.kernel == VK_LDS) {
+        if (plan.kernel == VK_MFMA_GEMM) {
+            e = vlut_launch_gemm(p, plan, s);
+        } else if (plan.kernel == VK_LDS) {
             e = p.q == 4 ? dispatch_m<4>(p, VLUT_METHOD_LDS, splits, s) : dispatch_m<2>(p, VLUT_METHOD_LDS, splits, s);
         } else if (!p.swar_ok) {
             return hipErrorInvalidValue;
@@ -1264,8 +1312,9 @@ hipError_t vlut_matmul(VlutMatmulArgs p, const VlutPlan& plan, hipStream_t s)
             hipLaunchKernelGGL(vlut_reduce_planes4_kernel,
                                dim3((unsigned)((p.rows + 63) / 64), (unsigned)((p.planes_b + 15) / 16)), dim3(256), 0, s, p.partial, splits, p.planes_b, p.rows, p.scale, p.scale_mode, mult,
                                p.bias, p.lsq_alpha, p.lsq_qmax, p.out);
-        } else if (v4 && plan.kernel == VK_MFMA_DEEP) {
-            hipLaunchKernelGGL(vlut_reduce_rg4_kernel, dim3((unsigned)((p.rows + 63) / 64), (unsigned)((p.B + 15) / 16)),
+        } else if (v4 && (plan.kernel == VK_MFMA_DEEP || plan.kernel == VK_MFMA_GEMM)) {
+            auto* reduce = plan.kernel == VK_MFMA_GEMM ? vlut_reduce_rg4_kernel<true> : vlut_reduce_rg4_kernel<false>;
+            hipLaunchKernelGGL(reduce, dim3((unsigned)((p.rows + 63) / 64), (unsigned)((p.B + 15) / 16)),
                                dim3(256), 0, s, p.partial, splits, p.B, p.rows, p.scale, p.scale_mode, mult, p.bias,
                                p.lsq_alpha, p.lsq_qmax, p.out);
         } else if (v4 && plan.kernel == VK_LDS)
@@ -1285,10 +1334,12 @@ hipError_t vlut_matmul(VlutMatmulArgs p, const VlutPlan& plan, hipStream_t s)
             hipLaunchKernelGGL(vlut_reduce_sm4_kernel, dim3((unsigned)((nw / 4 + 255) / 256)), dim3(256), 0, s,
                                p.partial, splits, p.B, p.rows, p.scale, p.scale_mode, mult, p.bias, p.lsq_alpha,
                                p.lsq_qmax, p.out);
-        else
-            hipLaunchKernelGGL(vlut_reduce_sm_kernel, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, s, p.partial,
+        else {
+            auto* reduce = plan.kernel == VK_MFMA_GEMM ? vlut_reduce_sm_kernel<true> : vlut_reduce_sm_kernel<false>;
+            hipLaunchKernelGGL(reduce, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, s, p.partial,
                                splits, p.B, p.rows, p.scale, p.scale_mode, mult, p.bias, p.lsq_alpha, p.lsq_qmax,
                                p.out);
+        }
         return hipGetLastError();
     }
     if (plan.kernel == VK_MFMA_ROWS) {

@@ -131,9 +131,8 @@ VlutPlan vlut_plan(int64_t rows, int64_t B, int64_t K, int q, int M, int method,
 // kernel runs unsplit and writes the output itself.
 inline int64_t vlut_workspace_floats(const VlutPlan& plan, int64_t B, int64_t rows)
 {
-    if (plan.kernel == VK_MFMA_GEMM) return 0;
     if ((plan.kernel == VK_MFMA_ROWS || plan.kernel == VK_MFMA_WIDE || plan.kernel == VK_MFMA_DEEP ||
-         plan.kernel == VK_LDS) &&
+         plan.kernel == VK_MFMA_GEMM || plan.kernel == VK_LDS) &&
         plan.splits == 1)
         return 0;
     return (int64_t)plan.splits * B * rows;

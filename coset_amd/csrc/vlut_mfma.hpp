@@ -212,9 +212,12 @@ hipError_t vlut_launch_rows(const VlutMatmulArgs& p, int splits, hipStream_t s);
 bool vlut_rows_staged(int64_t K, int splits);
 hipError_t vlut_launch_wide(const VlutMatmulArgs& p, int splits, hipStream_t s);
 hipError_t vlut_launch_deep(const VlutMatmulArgs& p, int splits, hipStream_t s);
-// The GEMM kernel of the decoded formats (vlut_gemm.hip) in tile shape
-// `shape`, and the shape the plan takes for these sizes (-1: the deep kernel).
-hipError_t vlut_launch_gemm(const VlutMatmulArgs& p, int shape, hipStream_t s);
-int vlut_gemm_shape(int64_t rows, int64_t B, int64_t K, int cus);
+// The GEMM kernel of the decoded formats (vlut_gemm.hip): fp16, bf16 or, with
+// shapes of their own, fp32 activations; splits > 1 writes split-major partials
+// and leaves the reduce to the caller.  The plans: kernel VK_MFMA_GEMM, or
+// VK_MFMA_DEEP where the deep kernel is faster.
+hipError_t vlut_launch_gemm(const VlutMatmulArgs& p, const VlutPlan& plan, hipStream_t s);
+VlutPlan vlut_gemm_plan(int64_t rows, int64_t B, int64_t K, int cus);
+VlutPlan vlut_gemm32_plan(int64_t rows, int64_t B, int64_t K, int cus, int64_t max_splits);
 
 }  // namespace coset

@@ -20,7 +20,7 @@ def _weight(rows, K, q, M, seed):
 
 
 @pytest.mark.parametrize("layout", ["decoded", "decoded6"])
-@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape", [0, 1, 2, 3])
 @pytest.mark.parametrize("B,rows,K", [(1, 4, 8), (129, 40, 64), (257, 200, 72), (300, 259, 1064), (127, 193, 200)])
 def test_gemm_shapes_vs_dense(layout, dt, shape, B, rows, K):
@@ -110,3 +110,50 @@ def test_gemm_under_graph_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("B,rows,K", [(48, 768, 3072), (49, 132, 2056), (200, 1000, 1000), (64, 130, 4096)])
+def test_gemm_fp32_splits(B, rows, K):
+    """fp32 activations over a wide range of magnitudes through the natural
+    plan (many K splits at few tokens; rows % 4 != 0 takes the scalar reduce),
+    with bias: within the fp32 bound, and no further from float64 than the three
+    planes run as 3B tokens on the deep kernel (times 1.25: both are rounding
+    noise)."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    words, W, g = _weight(rows, K, 4, 2, B)
+    w = ca.vlut_prepare(words, 4, layout="decoded")
+    a = torch.randn(B, K, device="cuda", generator=g)
+    a *= torch.exp2(torch.randint(-6, 7, (B, 1), device="cuda", generator=g).float())
+    sc = torch.rand(rows, device="cuda", generator=g) + 0.5
+    bias = torch.randn(rows, device="cuda", generator=g)
+    ref = (a.double() @ W.t()) * sc + bias
+    mag = (a.double().abs() @ W.t().abs()) * sc + bias.abs()
+    y = ca.vlut_matmul(w, a, scale=sc, bias=bias)
+    try:
+        _lib.set_vlut_gemm(0)
+        y0 = ca.vlut_matmul(w, a, scale=sc, bias=bias)
+    finally:
+        _lib.set_vlut_gemm(1)
+    assert ((y - ref).abs() <= RTOL * mag).all()
+    assert (y - ref).norm() <= 1.25 * (y0 - ref).norm()
+
+
+def test_gemm_fp32_special_values():
+    """Infinities and NaN stay in their token, and an output is finite exactly
+    where the deep kernel's is."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    words, W, g = _weight(768, 3072, 4, 2, 8)
+    w = ca.vlut_prepare(words, 4, layout="decoded6")
+    a = torch.randn(60, 3072, device="cuda", generator=g)
+    a[3, 5], a[9, 3071], a[20, 100], a[30] = float("inf"), -float("inf"), float("nan"), 1e-40
+    y = ca.vlut_matmul(w, a)
+    try:
+        _lib.set_vlut_gemm(0)
+        y0 = ca.vlut_matmul(w, a)
+    finally:
+        _lib.set_vlut_gemm(1)
+    assert torch.equal(torch.isfinite(y), torch.isfinite(y0))
+    keep = [i for i in range(60) if i not in (3, 9, 20)]
+    assert torch.isfinite(y[keep]).all()
