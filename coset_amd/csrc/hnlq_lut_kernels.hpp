@@ -38,9 +38,9 @@ constexpr int kLutThreads = 1024;
 // counter ring (counters.hpp) for each launch -- [0] hands out tiles, [1]
 // counts finished workgroups, and the workgroup that finishes last puts both
 // back to zero and then releases the slot to the host.
-constexpr int kTileBlocks = 2;        // blocks per thread in a dynamic tile
+constexpr int kTileBlocks = 2;        // blocks per thread in a dynamic tile (1 where float codes are written)
 constexpr int64_t kDynamicMinBlocks = 3 << 21;   // the fp32 round trip takes its tiles from a counter from here on
-
+constexpr int64_t kDynamicMinBlocksCodes = 1 << 21;   // the same where float codes are written
 
 // Copies the decode tables to LDS: the map (n_map uint4) and the byte or
 // coarse table (n_tab uint64).  Each thread issues all its loads before any
@@ -147,41 +147,56 @@ __device__ __forceinline__ void tiles_done(unsigned* tiles, unsigned* release)
     }
 }
 
-// Dynamic tiles of two blocks per thread, blockDim.x apart, with one block
+// Dynamic tiles of KT blocks per thread, blockDim.x apart, with one block
 // ahead; one LDS barrier per tile.
-template <typename In, typename Load, typename Body>
+template <int KT, typename In, typename Load, typename Body>
 __device__ __forceinline__ void schedule_tiles(int64_t n, TileCounters tc, unsigned* s_tile, Load& load, Body& body)
 {
+    static_assert(KT == 1 || KT == 2, "register sets alternate per block");
     unsigned* tiles = tc.pair;
     const int64_t last = n - 1;
-    const int64_t ntiles = (n + kTileBlocks * (int64_t)blockDim.x - 1) / (kTileBlocks * (int64_t)blockDim.x);
+    const int64_t ntiles = (n + KT * (int64_t)blockDim.x - 1) / (KT * (int64_t)blockDim.x);
     auto blk = [&](int64_t t, int j) {
-        const int64_t b = (t * kTileBlocks + j) * blockDim.x + threadIdx.x;
+        const int64_t b = (t * KT + j) * blockDim.x + threadIdx.x;
         return b < n ? b : last;
     };
     const int64_t t0 = blockIdx.x;
     int64_t t1 = t0 + gridDim.x;
     In in0, in1;
-    auto tile = [&](int64_t cur, int64_t nxt, int slot) {
-        load(blk(cur, 1), in1);
-        body(blk(cur, 0), in0);
+    // s0 holds the tile's first block; with KT == 1 the next tile's starts in s1, else in s0
+    auto tile = [&](int64_t cur, int64_t nxt, In& s0, In& s1, int slot) {
+        if constexpr (KT == 2) {
+            load(blk(cur, 1), s1);
+            body(blk(cur, 0), s0);
+        }
+        In& now = KT == 2 ? s1 : s0;
+        In& ahead = KT == 2 ? s0 : s1;
         unsigned grab = 0;
         if (threadIdx.x == 0) grab = atomicInc(tiles, ~0u);
-        load(blk(nxt, 0), in0);
-        body(blk(cur, 1), in1);
+        load(blk(nxt, 0), ahead);
+        body(blk(cur, KT - 1), now);
         if (threadIdx.x == 0) s_tile[slot] = grab;
         lds_barrier();
         return (int64_t)s_tile[slot] + 2 * (int64_t)gridDim.x;
     };
     if (t0 < ntiles) {
         load(blk(t0, 0), in0);
-        int64_t t2 = tile(t0, t1, 0);
-        int slot = 1;
-        while (t1 < ntiles) {
-            const int64_t t3 = tile(t1, t2, slot);
-            slot ^= 1;
-            t1 = t2;
-            t2 = t3;
+        int64_t t2 = tile(t0, t1, in0, in1, 0);
+        if constexpr (KT == 1) {
+            while (t1 < ntiles) {
+                const int64_t t3 = tile(t1, t2, in1, in0, 1);
+                if (t2 >= ntiles) break;
+                t1 = t3;
+                t2 = tile(t2, t3, in0, in1, 0);
+            }
+        } else {
+            int slot = 1;
+            while (t1 < ntiles) {
+                const int64_t t3 = tile(t1, t2, in0, in1, slot);
+                slot ^= 1;
+                t1 = t2;
+                t2 = t3;
+            }
         }
     }
     tiles_done(tiles, tc.release);
@@ -518,13 +533,16 @@ __global__ void __launch_bounds__(kLutThreads) hnlq_plain_kernel(CodecArgs a, co
     constexpr int NC = LutShape<Q>::kCodes;
     __shared__ __align__(16) uint16_t s_map[NC];
     __shared__ uint64_t s_tab[512 + kMaxCoarse];
-    // tiles from a counter in the fp32 round trip only: the counter hands out one
+    // tiles from a counter in the fp32 round trip and where float codes are written: the counter hands out one
     // tile per ~13 ns whatever the tile holds, which the shorter bodies wait
     // for (bf16 decode of 2^24 blocks: 106 us from the counter, 53 with the grid
     // stride; encode 165 / 157), and its hand-back at the end costs 2-4 us
     // (kDynamicMinBlocks: round trip of 2^22 blocks 52.5 / 50.5, of 2^23 98.7 /
-    // 107.7, of 2^24 203 / 227)
-    constexpr bool kDynamic = MODE == MODE_ROUNDTRIP && !XBF && !OBF;
+    // 107.7, of 2^24 203 / 227).  Float codes are 64 bytes of stores a block, whose
+    // speed differs between workgroups (kDynamicMinBlocksCodes, tiles of one block
+    // per thread): encode of 2^20 blocks 20.2 / 19.0, of 2^21 34.3 / 37.3, of 2^24
+    // 263 / 322; round trip 26.7 / 25.3, 44.9 / 46.8, 368 / 432
+    constexpr bool kDynamic = CODES || (MODE == MODE_ROUNDTRIP && !XBF && !OBF);
     __shared__ unsigned s_tile[kDynamic ? 2 : 1];
     __shared__ float4 s_stage[MODE == MODE_ENCODE && !CODES ? 1 : kLutThreads / 64][64];  // store_*_wave
     auto stage = [&]() {
@@ -738,7 +756,7 @@ __global__ void __launch_bounds__(kLutThreads) hnlq_plain_kernel(CodecArgs a, co
     // every store of a body is unconditional (see the schedules above)
     if constexpr (kDynamic) {
         if (tc.pair) {
-            schedule_tiles<In>(n, tc, s_tile, load, body);
+            schedule_tiles<CODES ? 1 : kTileBlocks, In>(n, tc, s_tile, load, body);
             return;
         }
     }
@@ -772,7 +790,8 @@ hipError_t launch_plain(const CodecArgs& a, int grid, const uint16_t* map, const
         const bool codes = MODE != MODE_DECODE && a.codes_f32;
         const bool xbf = MODE != MODE_DECODE && a.x_dtype == DT_BF16, obf = MODE != MODE_ENCODE && a.out_dtype == DT_BF16;
         const bool div = a.scale_mode == SCALE_CODEC && !a.beta_is_pow2;
-        const TileCounters tiles = g_codec_dynamic && MODE == MODE_ROUNDTRIP && !xbf && !obf && a.n >= kDynamicMinBlocks
+        const bool dynamic = codes || (MODE == MODE_ROUNDTRIP && !xbf && !obf);
+        const TileCounters tiles = g_codec_dynamic && dynamic && a.n >= (codes ? kDynamicMinBlocksCodes : kDynamicMinBlocks)
                                        ? take_counters(s)
                                        : TileCounters{nullptr, nullptr, -1};
         // packed words are always written by the encoder, optional in the

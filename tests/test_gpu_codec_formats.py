@@ -116,3 +116,31 @@ def test_sizes_around_the_dispatch_lines(n):
     s = torch.int16
     assert torch.equal(got[0].view(s), want[0].view(s)) and torch.equal(words.view(s), want[0].view(s))
     assert torch.equal(got[1], want[1]) and torch.equal(dec, want[1])
+
+
+@pytest.mark.parametrize("q,M", [(4, 2), (2, 3)])
+@pytest.mark.parametrize("n", [1 << 21, (1 << 21) + 1, (1 << 21) + 1023 * 1024 + 3, (3 << 20) + 1025])
+def test_float_codes_from_the_tile_counter(q, M, n):
+    """Encode and round trip with float codes from their counter line on
+    (tiles of one block per thread), last tiles full and ragged: bit for bit
+    the grid stride's outputs, every element written."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    x = _x(n, 11)
+    out = []
+    try:
+        for dynamic in (True, False):
+            _lib.set_codec_dynamic(dynamic)
+            rt = torch.full((n, M), -1, dtype=torch.int16, device="cuda")
+            rc = torch.full((n, M, 8), -1.0, device="cuda")
+            dec = torch.full((n, 8), float("nan"), device="cuda")
+            w, c = ca.hnlq_encode(x, q, M, None, return_codes=True)
+            _lib.call("coset_e8_hnlq_roundtrip", x.data_ptr(), _lib.F32, n, _lib.SCALE_NONE, 1.0, None, 0, 0.0, None, 0,
+                      q, M, 1, rt.data_ptr(), rc.data_ptr(), dec.data_ptr(), _lib.F32, _lib.stream_of(x))
+            out.append((w.view(torch.int16), c, rt, rc, dec))
+    finally:
+        _lib.set_codec_dynamic(True)
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    assert torch.equal(out[0][0], out[0][2]) and torch.equal(out[0][1], out[0][3])
+    assert (out[0][3] >= 0).all() and torch.isfinite(out[0][4]).all()
