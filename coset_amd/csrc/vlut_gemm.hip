@@ -22,9 +22,9 @@
 // the latency of the stages (0.9 us each, 64 x 64 tiles) and of the reduce.
 //
 // Bound: at 4096 x 4096 x 4096 tokens 1148 TFLOP/s (bf16, 256 x 256 tiles over the whole K), the matrix cores at
-// the clock the chip holds under them; at 3072 x 768 x 4096 tokens 29.3 us, of
-// which the 50 MB of fp32 output take 10 (the deep kernel, which decodes each
-// weight for 64 tokens, takes 90.5).  Decoding at the store to LDS costs one
+// the clock the chip holds under them; at 3072 x 768 x 4096 tokens 38 us on the plan's
+// 128 x 128 tiles (kOneChainK), of which the 50 MB of fp32 output take 10 (the deep
+// kernel, which decodes each weight for 64 tokens, takes 104).  Decoding at the store to LDS costs one
 // decode per BT tokens, 20 VALU operations per 8 weights in bf16.  Waves in
 // two groups a phase apart (one loads while the other multiplies) measured the
 // same at full load and slower on the smaller shapes; 4 waves of 128 x 128
@@ -346,7 +346,11 @@ struct GemmShape {
     int bt, br;
     double stage_us, fixed_us;
 };
-constexpr int64_t kOneChainK = 1024;   // the most K summed in one chain
+// The most K that the 256-token tiles, whose sums are one chain, take: above,
+// their error against 64 bits is larger than the deep kernel's (fp16, 1000 K
+// 7.7e-8 against 6.7e-8, 128 x 128 tiles 6.5e-8; bf16, 768 K 5.1e-8, 5.0e-8,
+// 5.0e-8), though 4096 tokens of 3072 x 768 take 29 us on them and 38 on 128 x 128
+constexpr int64_t kOneChainK = 256;
 constexpr GemmShape kGemmShapes[] = {{256, 256, 1.51, 8.3}, {256, 192, 1.26, 8.1}, {128, 128, 0.59, 4.1},
                                      {128, 64, 0.42, 3.5}};
 
@@ -422,7 +426,7 @@ VlutPlan vlut_gemm_plan(int64_t rows, int64_t B, int64_t K, int cus)
     // workgroup per CU (its phases do not overlap), 1.5 us for the reduce of
     // its splits.  bf16, us, deep / this kernel: 768 x 3072 x 256 tokens (the
     // splits fill the chip) 12.0 / 12.9, x 512 18.6 / 15.6, x 1024 28.5 / 20.3; 3072 x 768 x 256
-    // 9.3 / 8.8, x 4096 90.5 / 29.3; 4096 x 4096 x 256 34.0 / 31.2, x 4096 557 /
+    // 9.3 / 8.8, x 4096 103.9 / 38.1; 4096 x 4096 x 256 34.0 / 31.2, x 4096 557 /
     // 157 on 128 x 128 tiles (120 on 256 x 256, which sum 4096 K in one chain)
     const int64_t kq = (K / 8 + 3) / 4;
     const int64_t groups = ((rows + kDeepRows - 1) / kDeepRows) * ((B + kDeepTokens - 1) / kDeepTokens);
