@@ -493,6 +493,16 @@ def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: b
     need_db = need_db and bias_dtype is not None
     g2 = gy.reshape(-1, gy.shape[-1])
     dx = dW = db = None
+    if torch.is_grad_enabled():
+        # a backward with create_graph=True: torch's products and sums, which
+        # autograd can differentiate again (the kernels below leave no graph)
+        if need_dx:
+            dx = (g2 @ Wq).reshape(x.shape)
+        if need_dw:
+            dW = g2.t() @ x.reshape(-1, x.shape[-1])
+        if need_db:
+            db = g2.float().sum(0).to(bias_dtype)
+        return dx, dW, db
     fast_db = (need_db and g2.shape[1] % 8 == 0
                and g2.dtype in (torch.float32, torch.bfloat16, torch.float16))
     overlap = g2.is_cuda and (_OVERLAP_BACKWARD[0] > 0 or torch.cuda.is_current_stream_capturing())
