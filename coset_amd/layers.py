@@ -585,12 +585,30 @@ class QATLinearFn(torch.autograd.Function):
         return (*linear_grads(gy, x, Wq, ctx.bias_dtype, need[0], need[1], need[2]), None)
 
 
+class _AttachedWeight(torch.autograd.Function):
+    """The W_q that a forward has saved, attached to the weight and theta it was
+    made from: E8ThetaWeightQuant without a second quantization."""
+
+    @staticmethod
+    def forward(ctx, W, theta, Wq, Wc, packed, beta, dbdt, cfg):
+        ctx.save_for_backward(Wc, packed, beta, dbdt)
+        ctx.cfg = cfg
+        return Wq.detach()
+
+    @staticmethod
+    def backward(ctx, g):
+        dW, dtheta = qat_bwd_theta(g, *ctx.saved_tensors, *ctx.cfg)
+        return dW, dtheta, None, None, None, None, None, None
+
+
 class QATLayerFn(torch.autograd.Function):
     """The fused layer as one autograd node: W_q as E8ThetaWeightQuant makes it,
     y = x W_q^T + b as QATLinearFn does, and both backwards in turn.  cfg:
     (bounds, q, M, clip, blocks_per_tile).  Half the nodes of the two functions
     one after the other, whose Python and engine overhead an eager step of a
-    small batch waits for."""
+    small batch waits for.  W and theta are leaves (the layer's parameters, or a
+    buffer): a backward that autograd records reaches them through the saved
+    W_q, as it does through the two functions."""
 
     @staticmethod
     def forward(ctx, x, W, theta, bias, sigma, xmax, step_count, cfg):
@@ -601,6 +619,7 @@ class QATLayerFn(torch.autograd.Function):
         Wq, packed, beta, dbdt, b_cast = qat_fwd_theta(Wc, theta.detach(), sigma, xmax, step_count, bounds, q, M, clip,
                                                        bpt, x.dtype, bias if cast else None)
         ctx.save_for_backward(x, Wq, Wc, packed, beta, dbdt)
+        ctx.leaves = (W, theta)   # for their place in the graph only: the values are in what is saved
         ctx.cfg = (q, M, clip, bpt, theta.shape)
         ctx.bias_dtype = None if bias is None else bias.dtype
         if bias is not None and b_cast is None:
@@ -610,6 +629,8 @@ class QATLayerFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gy):
         x, Wq, Wc, packed, beta, dbdt = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            Wq = _AttachedWeight.apply(*ctx.leaves, Wq, Wc, packed, beta, dbdt, ctx.cfg)
         need = ctx.needs_input_grad
         dx, dWq, db = linear_grads(gy, x, Wq, ctx.bias_dtype, need[0], need[1] or need[2], need[3])
         dW = dtheta = None
@@ -907,7 +928,7 @@ class HNLQLinearQAT(nn.Module):
         if self._head_takes(x):
             return self._head_forward(x)
         if (x.is_cuda and self.quantization_enabled and not self.enable_diagnostics and self._fused()
-                and x.dtype in (torch.float32, torch.bfloat16)):
+                and x.dtype in (torch.float32, torch.bfloat16) and self.weight.is_leaf and self.theta_beta.is_leaf):
             self._advance_step(device_increment=False)   # the kernel increments step_count
             bpt = self.blocks_per_row if self.tiling == "row" else 1
             x = QATLayerFn.apply(x, self.weight, self.theta_beta, self.bias, self.sigma_ema, self.xmax_ema,
