@@ -51,3 +51,37 @@ def test_in_place_weight_update_is_caught():
         layer.weight.mul_(2.0)
     with pytest.raises(RuntimeError):
         y.sum().backward()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("how", ["subclass", "instance"])
+def test_overridden_weight_quantizer_is_called(dt, how):
+    """A replaced weight quantizer (a subclass's method or one set on the
+    layer) decides the weight of the training forward, and its gradient."""
+    import types
+    import coset_amd as ca
+    from coset_amd.layers import HNLQLinearQAT
+
+    class Halved(HNLQLinearQAT):
+        def _quantize_weights_with_bias(self, out_dtype, cast_bias):
+            W_q, b = super()._quantize_weights_with_bias(out_dtype, cast_bias)
+            return W_q * 0.5, b
+
+    torch.manual_seed(1)
+    plain = ca.create_e8_hnlq_linear(72, 40, Delta0=1.5)
+    layer = ca.create_e8_hnlq_linear(72, 40, Delta0=1.5)
+    layer.load_state_dict(plain.state_dict())
+    if how == "subclass":
+        layer.__class__ = Halved
+    else:
+        def halved(self, out_dtype, cast_bias):
+            W_q, b = HNLQLinearQAT._quantize_weights_with_bias(self, out_dtype, cast_bias)
+            return W_q * 0.5, b
+        layer._quantize_weights_with_bias = types.MethodType(halved, layer)
+    x = torch.randn(33, 72, device="cuda").to(dt)
+    y0, y = plain(x), layer(x)
+    with torch.no_grad():
+        assert torch.equal(y, y0 * 0.5)        # halving is exact; the bias is zero
+    y0.sum().backward()
+    y.sum().backward()
+    assert torch.equal(layer.weight.grad, 0.5 * plain.weight.grad)
