@@ -231,7 +231,10 @@ def set_vlut_deep(enabled: bool) -> None:
 def set_vlut_gemm(mode: int) -> None:
     """Large vLUT batches of the decoded formats: 0 the deep kernel, 1 the
     GEMM kernel where the plan prefers it (default), 2 + s its tile shape s
-    (256 x 256, 256 x 192, 128 x 128 or 128 x 64 tokens x rows) always."""
+    always, at any batch: 256 x 256, 256 x 192, 128 x 128 or 128 x 64 tokens x
+    rows, for fp32 activations 128 x 128, 64 x 128, 64 x 64 or 64 x 64.  Without
+    effect where the byte-table decode or the deep kernel is switched off or K
+    splits are forced."""
     call("coset_set_option", OPT_VLUT_GEMM, int(mode))
 
 

@@ -790,9 +790,10 @@ static int vlut_matmul_impl(const void* words, int word_format, const float* sca
     if (!words || !act || !out) return fail(COSET_EINVAL, "NULL buffer");
     if (!aligned(act, 16) || !aligned(words, 4)) return fail(COSET_EINVAL, "act must be 16-byte aligned, words 4-byte");
     const bool split = m == coset::VLUT_METHOD_MFMA_SPLIT;
-    // the split path's inner product: 3B bf16 tokens on the matrix cores
-    const coset::VlutPlan plan = coset::vlut_plan(rows, split ? 3 * B : B, K, q, M, split ? coset::VLUT_METHOD_MFMA : m,
-                                                   word_format);
+    // the split path's inner product: 3B bf16 tokens on the matrix cores (never
+    // the GEMM kernel, which takes fp32 activations whole: vlut_matmul_split)
+    const coset::VlutPlan plan = split ? coset::vlut_plan(rows, 3 * B, K, q, M, coset::VLUT_METHOD_MFMA)
+                                       : coset::vlut_plan(rows, B, K, q, M, m, word_format);
     const int64_t need = vlut_method_workspace(m, B, rows, K, q, M);
     if (workspace_floats < need)
         return fail(COSET_EINVAL, "workspace holds %lld floats, needs %lld", (long long)workspace_floats,

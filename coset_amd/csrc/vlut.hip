@@ -1187,8 +1187,14 @@ __global__ void __launch_bounds__(256) vlut_split_sum_kernel(const float* __rest
 
 namespace {
 
-// Tokens from which fp32 activations take the GEMM kernel's own split
-constexpr int64_t kGemm32Tokens = 48;
+// Tokens from which fp32 activations take the GEMM kernel's own split: where
+// their three planes need a third token tile of the deep kernel.  43 tokens, us,
+// planes on the deep kernel / split here, rows x K: 768 x 3072 17.4 / 14.5, 3072 x
+// 768 13.4 / 10.5, 1000 x 1000 16.6 / 10.5, 4096 x 1000 13.7 / 12.5, 4096 x 4096
+// 28.4 / 19.6, 256 x 256 15.7 / 6.6; error against 64 bits at 4096 K 6.1e-8 /
+// 4.1e-8.  At 42 the planes take 19.3, 12.4, 19.5, 12.6, 23.5 and 15.6.
+constexpr int64_t kGemm32Tokens = 43;
+static_assert(3 * (kGemm32Tokens - 1) <= 2 * kDeepTokens && 3 * kGemm32Tokens > 2 * kDeepTokens, "two deep token tiles");
 
 constexpr int64_t align64(int64_t n) { return (n + 63) / 64 * 64; }
 
@@ -1211,7 +1217,7 @@ hipError_t vlut_matmul_split(VlutMatmulArgs p, float* workspace, hipStream_t s)
     q.act_dtype = DT_BF16;
     q.B = 3 * B;
     q.partial = inner;
-    const VlutPlan plan = vlut_plan(p.rows, 3 * B, p.K, p.q, p.M, VLUT_METHOD_MFMA, p.prepared);
+    const VlutPlan plan = vlut_plan(p.rows, 3 * B, p.K, p.q, p.M, VLUT_METHOD_MFMA);
     // the plane sum goes into the plan's last kernel where that kernel holds
     // all three planes of an output: the rows kernel with one split and one
     // token tile, or the reduce of a split wide / deep kernel; a staged rows
@@ -1219,7 +1225,7 @@ hipError_t vlut_matmul_split(VlutMatmulArgs p, float* workspace, hipStream_t s)
     const bool v4 = p.rows % 4 == 0 && ((uintptr_t)p.out % 16) == 0 && ((uintptr_t)inner % 16) == 0;
     const bool rows1 = plan.kernel == VK_MFMA_ROWS && plan.splits == 1;
     if ((p.prepared == VLUT_DECODED || p.prepared == VLUT_DECODED6) && g_vlut_deep && g_vlut_gemm && g_vlut_swar &&
-        g_vlut_splits == 0 && B >= kGemm32Tokens) {
+        g_vlut_splits == 0 && (B >= kGemm32Tokens || g_vlut_gemm >= 2)) {
         // the GEMM kernel splits the fp32 activations itself, in one launch
         // and a reduce; its partials fit the workspace's splits
         const int64_t room = vlut_split_workspace_floats(B, p.rows, p.K, p.q, p.M) / std::max<int64_t>(1, B * p.rows);

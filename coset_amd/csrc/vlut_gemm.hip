@@ -15,7 +15,7 @@
 // first operand, so a lane ends with 4 consecutive output rows of one token.  The loads of stage s + 2 go out while stage s is
 // multiplied and their data is stored to LDS in the middle of stage s + 1.
 //
-// fp32 activations (from 48 tokens): one launch and a reduce, where the planes
+// fp32 activations (from 43 tokens): one launch and a reduce, where the planes
 // took a split launch, 3B tokens on the deep kernel and a reduce: 197 tokens of
 // 768 x 3072 26.6 -> 17.5 us, 48 of 3072 x 768 13.5 -> 10.6, 4096 of 3072 x 768
 // 306 -> 86; error against 64 bits 6.1e-8 -> 4.6e-8.  At few tokens the time is

@@ -87,7 +87,10 @@ enum {
     COSET_OPT_CODEC_DYNAMIC = 6,   /* fixed-format table kernel: 1 tiles from a counter run per launch (default), 0 grid stride */
     COSET_OPT_VLUT_DEEP = 7,       /* vLUT matmul above 32 tokens: 1 the 64-row deep kernel (default), 0 the 128-row wide one */
     COSET_OPT_GEMM_TN_TILE = 8,    /* coset_gemm_tn output tiles: 0 64 x 64 where they fit, else 96 x 96 (default); 64 or 96 only that size */
-    COSET_OPT_VLUT_GEMM = 9,       /* large vLUT batches of the decoded formats: 0 the deep kernel, 1 the GEMM kernel where the plan prefers it (default), 2..5 its tile shape 0..3 always */
+    COSET_OPT_VLUT_GEMM = 9,       /* large vLUT batches of the decoded formats: 0 the deep kernel, 1 the GEMM kernel where the plan prefers it (default), 2..5 its tile shape 0..3 always, at any
+                                      batch: 256 x 256, 256 x 192, 128 x 128, 128 x 64 tokens x rows; fp32 activations 128 x 128,
+                                      64 x 128, 64 x 64, 64 x 64.  Without effect where COSET_OPT_VLUT_DECODE or COSET_OPT_VLUT_DEEP
+                                      is 0 or COSET_OPT_VLUT_SPLITS is forced */
     COSET_OPT_GEMM_WGRAD = 10      /* coset_gemm_wgrad output tiles: 1 the plan's choice (default), 2, 3: 192 x 192 or 128 x 128 always */
 };
 

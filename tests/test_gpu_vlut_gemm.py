@@ -157,3 +157,32 @@ def test_gemm_fp32_special_values():
     assert torch.equal(torch.isfinite(y), torch.isfinite(y0))
     keep = [i for i in range(60) if i not in (3, 9, 20)]
     assert torch.isfinite(y[keep]).all()
+
+
+@pytest.mark.parametrize("layout", ["decoded", "decoded6"])
+@pytest.mark.parametrize("rows,K", [(256, 256), (768, 768), (1000, 1000), (768, 3072)])
+def test_fp32_at_the_gemm_kernels_first_tokens(layout, rows, K):
+    """42 fp32 tokens (126 plane tokens) run as planes on the deep kernel; 43 to
+    48, whose planes would reach the GEMM kernel, run on it whole: a token's
+    output is then the same whatever the call's token count (one token tile, the
+    same K splits)."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    words, W, g = _weight(rows, K, 4, 2, rows)
+    w = ca.vlut_prepare(words, 4, layout=layout)
+    a = torch.randn(48, K, device="cuda", generator=g)
+    sc = torch.rand(rows, device="cuda", generator=g) + 0.5
+    bias = torch.randn(rows, device="cuda", generator=g)
+    ref = (a.double() @ W.t()) * sc + bias
+    mag = (a.double().abs() @ W.t().abs()) * sc + bias.abs()
+    y = {B: ca.vlut_matmul(w, a[:B], scale=sc, bias=bias) for B in (42, 43, 47, 48)}
+    try:
+        _lib.set_vlut_gemm(0)
+        deep = ca.vlut_matmul(w, a[:42], scale=sc, bias=bias)
+    finally:
+        _lib.set_vlut_gemm(1)
+    assert torch.equal(y[42], deep)
+    for B in (43, 47):
+        assert torch.equal(y[B], y[48][:B])
+    for B, v in y.items():
+        assert ((v - ref[:B]).abs() <= RTOL * mag[:B]).all()
