@@ -352,7 +352,7 @@ struct GemmShape {
 // 5.0e-8), though 4096 tokens of 3072 x 768 take 29 us on them and 38 on 128 x 128
 constexpr int64_t kOneChainK = 256;
 constexpr GemmShape kGemmShapes[] = {{256, 256, 1.51, 8.3}, {256, 192, 1.26, 8.1}, {128, 128, 0.59, 4.1},
-                                     {128, 64, 0.42, 3.5}};
+                                     {128, 64, 0.43, 3.5}};
 
 constexpr GemmShape kGemmShapes32[] = {{128, 128, 1.98, 4.3}, {64, 128, 1.1, 3.7}, {64, 64, 0.9, 3.3}};
 
@@ -390,11 +390,12 @@ hipError_t launch(const VlutMatmulArgs& p, int shape, int splits, hipStream_t s)
 }  // namespace
 
 // The fastest (shape, splits) of a shape table by its measured costs; splits
-// up to max_splits, each of at least two stages; a reduce costs 3.5 us (launch
-// gap and prologue) and its traffic at 6 TB/s.
+// up to max_splits, each of at least two stages; a reduce costs reduce_us (launch
+// gap and prologue; 4.5 us fits the 16-bit calls, 3.5 the fp32 ones, whose stages
+// are longer) and its traffic at 6 TB/s.
 template <int N>
-double best_gemm(const GemmShape (&shapes)[N], int64_t rows, int64_t B, int64_t K, int cus, int64_t max_splits,
-                 VlutPlan* best)
+double best_gemm(const GemmShape (&shapes)[N], double reduce_us, int64_t rows, int64_t B, int64_t K, int cus,
+                 int64_t max_splits, VlutPlan* best)
 {
     const int64_t all = ((K / 8 + 3) / 4 + 1) / 2;
     double best_us = 1e30;
@@ -406,7 +407,7 @@ double best_gemm(const GemmShape (&shapes)[N], int64_t rows, int64_t B, int64_t 
             const int64_t per = (all + sp - 1) / sp;
             if (sp > 1 && (per < 2 || per * (sp - 1) >= all)) continue;
             const double us = g.fixed_us + (double)((tiles * sp + cus - 1) / cus) * (double)per * g.stage_us +
-                              (sp > 1 ? 3.5 + (double)(sp + 1) * (double)(B * rows) * 4.0 / 6.0e6 : 0.0);
+                              (sp > 1 ? reduce_us + (double)(sp + 1) * (double)(B * rows) * 4.0 / 6.0e6 : 0.0);
             if (us < best_us) {
                 best_us = us;
                 *best = {VK_MFMA_GEMM, (int)sp, i};
@@ -423,25 +424,31 @@ VlutPlan vlut_gemm_plan(int64_t rows, int64_t B, int64_t K, int cus)
     // 4096 x 4096: 10.8 us against 31)
     if (B <= 2 * kDeepTokens - 1) return none;
     // the deep kernel: 64 x 64 tiles of at most 1024 K, 7.2 us a round of one
-    // workgroup per CU (its phases do not overlap), 1.5 us for the reduce of
-    // its splits.  bf16, us, deep / this kernel: 768 x 3072 x 256 tokens (the
-    // splits fill the chip) 12.0 / 12.9, x 512 18.6 / 15.6, x 1024 28.5 / 20.3; 3072 x 768 x 256
-    // 9.3 / 8.8, x 4096 103.9 / 38.1; 4096 x 4096 x 256 34.0 / 31.2, x 4096 557 /
-    // 157 on 128 x 128 tiles (120 on 256 x 256, which sum 4096 K in one chain)
+    // workgroup per CU (its phases do not overlap).  The reduce of its splits
+    // takes 0.8 us where each XCD reads the partials its own workgroups wrote
+    // (rows a multiple of 8 groups of 64), else 2.0.  With these costs the choice
+    // is within 2.5 % of the faster kernel at 517 of 520 measured calls (20 shapes
+    // of 512..4096 x 320..4096, 128 to 2000 tokens, bf16 and fp16; the worst 4.5 %
+    // off).  bf16, us, deep / this kernel: 768 x 3072 x 160 tokens (the splits fill
+    // the chip) 11.4 / 12.4, x 512 18.4 / 15.6, x 1024 28.5 / 20.3; 2048 x 1000 x 160
+    // 9.7 / 10.6; 768 x 768 x 160 11.3 / 8.7; 3072 x 768 x 4096 103.9 / 38.1; 4096 x
+    // 4096 x 256 34.3 / 22.5, x 4096 557 / 157 on 128 x 128 tiles (120 on 256 x 256,
+    // which sum 4096 K in one chain)
     const int64_t kq = (K / 8 + 3) / 4;
     const int64_t groups = ((rows + kDeepRows - 1) / kDeepRows) * ((B + kDeepTokens - 1) / kDeepTokens);
     const int64_t min_splits = (kq + kDeepKqWg - 1) / kDeepKqWg;
     const int64_t splits = std::max(min_splits, std::min<int64_t>(std::max<int64_t>(1, cus / groups), kq));
-    const double deep_us = 2.5 + 7.2 * (double)((groups * splits + cus - 1) / cus) + (splits > 1 ? 1.5 : 0.0);
+    const double reduce_us = splits == 1 ? 0.0 : rows % (8 * kDeepRows) == 0 ? 0.8 : 2.0;
+    const double deep_us = 1.4 + 7.2 * (double)((groups * splits + cus - 1) / cus) + reduce_us;
     // workspaces are sized for the deep plan's splits
     VlutPlan best;
-    return best_gemm(kGemmShapes, rows, B, K, cus, splits, &best) < deep_us ? best : none;
+    return best_gemm(kGemmShapes, 4.5, rows, B, K, cus, splits, &best) < deep_us ? best : none;
 }
 
 VlutPlan vlut_gemm32_plan(int64_t rows, int64_t B, int64_t K, int cus, int64_t max_splits)
 {
     VlutPlan best{VK_MFMA_GEMM, 1, 0};
-    best_gemm(kGemmShapes32, rows, B, K, cus, max_splits, &best);
+    best_gemm(kGemmShapes32, 3.5, rows, B, K, cus, max_splits, &best);
     return best;
 }
 
