@@ -418,17 +418,32 @@ def gemm_wgrad(a: torch.Tensor, b: torch.Tensor, out_dtype: Optional[torch.dtype
     return out
 
 
-def _gemm_wgrad_takes(g2: torch.Tensor, x2: torch.Tensor, with_bias: bool) -> bool:
-    """Whether _weight_grad runs g2^T x2 on coset_gemm_wgrad, where
-    coset_gemm_tn does not take it.  Its column sums come free, while
-    coset_colsum costs 6-23 us beside the library's product: with a bias
-    gradient it was faster at every measured shape of up to 3072 x 3072
-    outputs (16384 tokens x 768 x 3072: 88 against 149 + 14 us; 1000 x 768 x
-    768: 15.4 against 13.0 + 6.5) but large outputs of few tokens (269 x 3072 x
-    2048: 21.6 against 13.7 + 6.6).  Without one the library is up to 25 %
-    faster below about 3000 tokens (755 x 1536 x 1024: 14.2 against 15.2),
-    slower above (3672 x 320 x 768: 29.6 against 18.0).  Larger outputs
-    (4096 x 4096 x 4096: 126 against 162) stay with the library."""
+def _gemm_wgrad_takes(g2: torch.Tensor, x2: torch.Tensor, with_bias: bool, with_dx: bool = False) -> bool:
+    """Whether the layer runs g2^T x2 on coset_gemm_wgrad, where coset_gemm_tn
+    does not take it; with_bias: its column sums are wanted too, with_dx: the
+    step also computes dX.
+
+    The kernel's column sums come free, while coset_colsum costs 6-23 us beside
+    the library's product: with a bias gradient and no dX it was faster at every
+    measured shape of up to 3072 x 3072 outputs (1000 x 768 x 768: 15.4 against
+    13.0 + 6.5 us) but large outputs of few tokens (269 x 3072 x 2048: 21.6
+    against 13.7 + 6.6).  Without one the library is up to 25 % faster below
+    about 3000 tokens (755 x 1536 x 1024: 14.2 against 15.2), slower above (3672
+    x 320 x 768: 29.6 against 18.0).  Larger outputs (4096 x 4096 x 4096: 126
+    against 162) stay with the library.
+
+    With dX the line lies elsewhere: a captured step runs dX beside dW, where the
+    library's column sums are hidden and this kernel's workgroups, one per CU,
+    slow dX.  Captured steps, us, library / this kernel (tokens x in x out): 1024 x
+    1024 x 2048 58 / 69, 1408 x 3072 x 512 61 / 71, 2816 x 2048 x 1536 104 / 115, 4992
+    x 1000 x 1536 106 / 110; 2688 x 512 x 1536 59 / 58, 6016 x 1024 x 512 77 / 67,
+    9472 x 1024 x 1024 152 / 104, 13824 x 3072 x 768 271 / 221.  Over 370 of them the
+    rule is within 0.5 % of the faster side on average (12 % at worst).  Above 4.8 M
+    outputs the library wins at most token counts (9985 x 2048 x 3072 350 / 386;
+    eager, 8000 tokens 309 / 336).  Eager steps follow the same rule, since replays
+    equal them bit for bit; there the host sets the time (1000 x 768 x 1000: 220
+    us with this kernel, 237 with the library and coset_colsum).
+    """
     if not (_GEMM_TN[0] == 1 and g2.is_cuda and x2.device == g2.device and g2.dtype == x2.dtype == torch.bfloat16
             and g2.dim() == 2 and x2.dim() == 2 and g2.shape[0] == x2.shape[0]):
         return False
@@ -438,25 +453,20 @@ def _gemm_wgrad_takes(g2: torch.Tensor, x2: torch.Tensor, with_bias: bool) -> bo
         return False
     if K < (512 if M * N > 1 << 22 else 1) or (not with_bias and K < 3000):
         return False
+    if with_dx and (M * N > 4800000 or 1000 * (K - 2000) < M * N):
+        return False
     # gemm_wgrad copies what is not contiguous; a contiguous operand has to be aligned
     return not ((g2.is_contiguous() and g2.data_ptr() % 16) or (x2.is_contiguous() and x2.data_ptr() % 16))
 
 
-def _weight_grad(g2: torch.Tensor, x2: torch.Tensor, colsum: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """dW_q = g2^T x2: coset_gemm_tn or coset_gemm_wgrad where they apply (with
-    colsum: also the fp32 column sums of g2, the bias gradient, in the same
-    pass), else torch.mm (colsum must then be None)."""
+def _weight_grad_kernel(g2: torch.Tensor, x2: torch.Tensor, with_bias: bool, with_dx: bool):
+    """The function that computes dW_q = g2^T x2 on a kernel of the library
+    (with a colsum argument: also the fp32 column sums of g2, the bias gradient,
+    in the same pass), or None where torch.mm does.  The choice is the same in
+    eager and captured steps, whose gradients are equal bit for bit."""
     if _gemm_tn_takes(g2, x2):
-        out = gemm_tn(g2, x2, colsum=colsum)
-        if out is not None:
-            return out
-    if _gemm_wgrad_takes(g2, x2, colsum is not None):
-        out = gemm_wgrad(g2, x2, colsum=colsum)
-        if out is not None:
-            return out
-    if colsum is not None:
-        raise RuntimeError("column sums requested where no weight-gradient kernel runs")
-    return g2.t() @ x2
+        return gemm_tn
+    return gemm_wgrad if _gemm_wgrad_takes(g2, x2, with_bias, with_dx) else None
 
 
 # 1: no-grad forwards of small fp32 batches run as one fused launch
@@ -506,30 +516,46 @@ def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: b
     fast_db = (need_db and g2.shape[1] % 8 == 0
                and g2.dtype in (torch.float32, torch.bfloat16, torch.float16))
     overlap = g2.is_cuda and (_OVERLAP_BACKWARD[0] > 0 or torch.cuda.is_current_stream_capturing())
-    x2 = x.reshape(-1, x.shape[-1])
-    if overlap and need_dw and (need_dx or fast_db) and g2.dtype == Wq.dtype == x.dtype:
-        # dX (and the bias gradient where coset_gemm_tn does not take it)
+    overlap = overlap and need_dw and (need_dx or fast_db) and g2.dtype == Wq.dtype == x.dtype
+    if overlap:
+        g2 = g2.contiguous()
+    # the bias gradient in the weight-gradient kernel's pass where one runs
+    # (bf16): the column sums of gy with gy^T x
+    kernel = None
+    fuse = need_dw and fast_db and _FUSE_BIAS_GRAD[0] == 1 and g2.dtype == torch.bfloat16 and g2.is_contiguous()
+    if need_dw:
+        x2 = x.reshape(-1, x.shape[-1])
+        kernel = _weight_grad_kernel(g2, x2, fuse, need_dx)
+        fuse = fuse and kernel is not None
+        dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device) if fuse else None
+
+    def weight_grad():
+        if kernel is None:
+            return torch.mm(g2.t(), x2)
+        out = kernel(g2, x2, colsum=dbf)
+        if out is None:
+            raise RuntimeError(f"{kernel.__name__} refused a product it was chosen for")
+        return out
+
+    if overlap:
+        # dX (and the bias gradient where no weight-gradient kernel takes it)
         # on a second stream while dW runs on this one: the dW product
         # alone leaves CUs idle at these shapes (one 64 x 64 or 128 x 128
         # tile per CU or fewer).  Outputs are allocated here, on the
         # current stream, before the fork; the join comes before they are
         # returned.  Under graph capture the two streams become two
         # branches of the graph.
-        g2 = g2.contiguous()
-        fuse = (_FUSE_BIAS_GRAD[0] == 1 and fast_db and g2.dtype == torch.bfloat16
-                and (_gemm_tn_takes(g2, x2) or _gemm_wgrad_takes(g2, x2, True)))
         main = torch.cuda.current_stream(g2.device)
         aux = _aux_stream(g2.device)
         dx2 = torch.empty((g2.shape[0], Wq.shape[1]), dtype=g2.dtype, device=g2.device) if need_dx else None
         cs = _colsum_buffers(g2) if fast_db and not fuse else None
-        dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device) if fuse else None
         aux.wait_stream(main)
         with torch.cuda.stream(aux):
             if need_dx:
                 torch.mm(g2, Wq, out=dx2)
             if cs is not None:
                 _colsum_into(g2, *cs)
-        dW = _weight_grad(g2, x2, colsum=dbf)
+        dW = weight_grad()
         main.wait_stream(aux)
         if need_dx:
             dx = dx2.reshape(x.shape)
@@ -538,25 +564,15 @@ def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: b
         elif need_db:
             db = g2.float().sum(0).to(bias_dtype)
         return dx, dW, db
-    # one stream: the bias gradient in the weight-gradient kernel's pass
-    # where that kernel runs (bf16), the column sums of gy with gy^T x
-    if (_FUSE_BIAS_GRAD[0] == 1 and fast_db and need_dw and g2.dtype == torch.bfloat16 and g2.is_contiguous()
-            and (_gemm_tn_takes(g2, x2) or _gemm_wgrad_takes(g2, x2, True))):
-        dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device)
-        dW = _weight_grad(g2, x2, colsum=dbf)
+    if need_dw and fuse:
+        dW = weight_grad()
         db = dbf.to(bias_dtype)
-        if need_dx:
-            dx = (g2 @ Wq).reshape(x.shape)
-        return dx, dW, db
     if need_dx:
         dx = (g2 @ Wq).reshape(x.shape)
-    if need_dw:
-        dW = _weight_grad(g2, x2)
-    if need_db:
-        if g2.shape[1] % 8 == 0 and g2.dtype in (torch.float32, torch.bfloat16, torch.float16):
-            db = colsum(g2).to(bias_dtype)
-        else:
-            db = g2.float().sum(0).to(bias_dtype)
+    if need_dw and not fuse:
+        dW = weight_grad()
+    if need_db and not fuse:
+        db = (colsum(g2) if fast_db else g2.float().sum(0)).to(bias_dtype)
     return dx, dW, db
 
 

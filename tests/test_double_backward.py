@@ -34,7 +34,7 @@ def kernels(monkeypatch):
             return a.t() @ b
 
     monkeypatch.setattr(layers, "_gemm_tn_takes", lambda a, b: False)
-    monkeypatch.setattr(layers, "_gemm_wgrad_takes", lambda a, b, with_bias: True)
+    monkeypatch.setattr(layers, "_gemm_wgrad_takes", lambda a, b, with_bias, with_dx=False: True)
     monkeypatch.setattr(layers, "gemm_wgrad", wgrad)
     monkeypatch.setattr(layers, "colsum", lambda a: a.detach().float().sum(0))
 

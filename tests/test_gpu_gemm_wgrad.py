@@ -124,3 +124,42 @@ def test_captured_step_replays_the_kernel():
         torch.cuda.synchronize()
         assert torch.equal(layer.weight.grad, want[0]) and torch.equal(layer.bias.grad, want[1])
         torch.zeros(1 << 20, device="cuda")
+
+
+@pytest.mark.parametrize("tokens,fin,fout,need_x,kernel", [
+    (1000, 256, 264, True, False), (1024, 1024, 2048, True, False), (2071, 256, 264, True, True),
+    (2067, 256, 264, True, False), (8000, 3072, 2048, True, False), (5000, 320, 512, True, True),
+    (1000, 256, 264, False, True), (1500, 512, 320, False, True)])
+def test_rule_of_a_step_with_and_without_dx(tokens, fin, fout, need_x, kernel):
+    """Which product takes the weight gradient, told by the bits of its K splits: with dX to
+    compute, torch.mm below 2000 tokens and one more per 1000 outputs and for
+    outputs above 4.8 M, else the kernel; the captured step's replays equal the
+    eager step's gradients bit for bit on both sides of the line."""
+    import coset_amd as ca
+    torch.manual_seed(7)
+    layer = ca.create_e8_hnlq_linear(fin, fout, Delta0=1.5)
+    with torch.no_grad():
+        layer.weight.mul_(0.02)
+    x = torch.randn(tokens, fin, device="cuda").to(torch.bfloat16).requires_grad_(need_x)
+    gy = torch.randn(tokens, fout, device="cuda").to(torch.bfloat16)
+
+    def grads():
+        layer.zero_grad(set_to_none=True)
+        x.grad = None
+        layer(x).backward(gy)
+        return [layer.weight.grad, layer.theta_beta.grad, layer.bias.grad, x.grad]
+
+    want = grads()
+    try:
+        layers.set_gemm_tn(False)
+        library = grads()
+    finally:
+        layers.set_gemm_tn(True)
+    assert torch.equal(want[0], library[0]) == (not kernel)
+    step = ca.CapturedQATStep(layer, x.detach().clone().requires_grad_(need_x), gy.clone())
+    for _ in range(3):
+        step.step()
+        torch.cuda.synchronize()
+        got = [layer.weight.grad, layer.theta_beta.grad, layer.bias.grad, step.x.grad]
+        for a, r in zip(got, want):
+            assert (a is None) == (r is None) and (a is None or torch.equal(a, r))
