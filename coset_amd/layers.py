@@ -425,12 +425,15 @@ def _gemm_wgrad_takes(g2: torch.Tensor, x2: torch.Tensor, with_bias: bool, with_
 
     The kernel's column sums come free, while coset_colsum costs 6-23 us beside
     the library's product: with a bias gradient and no dX it was faster at every
-    measured shape of up to 3072 x 3072 outputs (1000 x 768 x 768: 15.4 against
-    13.0 + 6.5 us) but large outputs of few tokens (269 x 3072 x 2048: 21.6
-    against 13.7 + 6.6).  Without one the library is up to 25 % faster below
-    about 3000 tokens (755 x 1536 x 1024: 14.2 against 15.2), slower above (3672
-    x 320 x 768: 29.6 against 18.0).  Larger outputs (4096 x 4096 x 4096: 126
-    against 162) stay with the library.
+    measured shape of up to 4.8 M outputs (1000 x 768 x 768: 15.4 against 13.0 +
+    6.5 us; 4200 x 1536 x 3072: 58 against 69 + 11).  Above, its tiles fill the
+    chip's rounds badly: it keeps up to 2000 tokens (1000 x 2048 x 3072: 33 against
+    29 + 10; 8000: 147 against 117 + 13), or one full round of 192 x 192 tiles
+    (4200 x 3072 x 3072: 91 against 93 + 10), and nothing above 3072 x 3072 outputs
+    (1000 x 4096 x 3072: 58 against 38 + 10) or below 512 tokens of wide ones.
+    Without a bias gradient the library is up to 25 % faster below about 3000
+    tokens (755 x 1536 x 1024: 14.2 against 15.2), slower above (3672 x 320 x 768:
+    29.6 against 18.0), faster again from 4.8 M outputs.
 
     With dX the line lies elsewhere: a captured step runs dX beside dW, where the
     library's column sums are hidden and this kernel's workgroups, one per CU,
@@ -453,7 +456,10 @@ def _gemm_wgrad_takes(g2: torch.Tensor, x2: torch.Tensor, with_bias: bool, with_
         return False
     if K < (512 if M * N > 1 << 22 else 1) or (not with_bias and K < 3000):
         return False
-    if with_dx and (M * N > 4800000 or 1000 * (K - 2000) < M * N):
+    if with_dx and 1000 * (K - 2000) < M * N:
+        return False
+    if M * N > 4800000 and (with_dx or not with_bias
+                            or (K > 2000 and not 248 <= -(-M // 192) * -(-N // 192) <= 256)):
         return False
     # gemm_wgrad copies what is not contiguous; a contiguous operand has to be aligned
     return not ((g2.is_contiguous() and g2.data_ptr() % 16) or (x2.is_contiguous() and x2.data_ptr() % 16))

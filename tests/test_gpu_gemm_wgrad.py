@@ -129,12 +129,15 @@ def test_captured_step_replays_the_kernel():
 @pytest.mark.parametrize("tokens,fin,fout,need_x,kernel", [
     (1000, 256, 264, True, False), (1024, 1024, 2048, True, False), (2071, 256, 264, True, True),
     (2067, 256, 264, True, False), (8000, 3072, 2048, True, False), (5000, 320, 512, True, True),
-    (1000, 256, 264, False, True), (1500, 512, 320, False, True)])
+    (1000, 256, 264, False, True), (1500, 512, 320, False, True),
+    (1900, 3072, 2048, False, True), (5000, 3072, 2048, False, False), (5000, 2048, 3072, False, False),
+    (5000, 3072, 3072, False, True)])
 def test_rule_of_a_step_with_and_without_dx(tokens, fin, fout, need_x, kernel):
-    """Which product takes the weight gradient, told by the bits of its K splits: with dX to
-    compute, torch.mm below 2000 tokens and one more per 1000 outputs and for
-    outputs above 4.8 M, else the kernel; the captured step's replays equal the
-    eager step's gradients bit for bit on both sides of the line."""
+    """Which product takes the weight gradient, told by the bits of its K splits
+    and column sums: with dX to compute, torch.mm below 2000 tokens and one more
+    per 1000 outputs and for outputs above 4.8 M, without dX for these from 2000
+    tokens unless one round of tiles holds them, else the kernel; the captured
+    step's replays equal the eager step's gradients bit for bit on both sides."""
     import coset_amd as ca
     torch.manual_seed(7)
     layer = ca.create_e8_hnlq_linear(fin, fout, Delta0=1.5)
@@ -155,7 +158,7 @@ def test_rule_of_a_step_with_and_without_dx(tokens, fin, fout, need_x, kernel):
         library = grads()
     finally:
         layers.set_gemm_tn(True)
-    assert torch.equal(want[0], library[0]) == (not kernel)
+    assert (torch.equal(want[0], library[0]) and torch.equal(want[2], library[2])) == (not kernel)
     step = ca.CapturedQATStep(layer, x.detach().clone().requires_grad_(need_x), gy.clone())
     for _ in range(3):
         step.step()
