@@ -194,7 +194,7 @@ def qat_fwd_theta(Wc, theta, sigma, xmax, step_count, bounds, q, M, clip, blocks
     dbdt = torch.empty_like(beta)
     b_in = b_out = None
     if bias is not None:
-        b_in = bias.detach().float().contiguous()
+        b_in = bias if bias.dtype == torch.float32 and bias.is_contiguous() else bias.detach().float().contiguous()
         if b_in.numel() != rows:
             raise ValueError(f"bias must hold {rows} values")
         b_out = torch.empty(rows, dtype=out_dtype, device=dev)
@@ -221,7 +221,7 @@ def qat_bwd_theta(g, Wc, packed, beta, dbdt, q, M, clip, blocks_per_tile, theta_
               g.data_ptr(), _lib.dtype_code(g.dtype), Wc.data_ptr(), packed.data_ptr(), beta.data_ptr(),
               dbdt.data_ptr(), rows, cols, blocks_per_tile, clip, q, M, dW.data_ptr(), dbeta.data_ptr(),
               dtheta.data_ptr(), _lib.stream_of(Wc))
-    return dW, dtheta.view(theta_shape)
+    return dW, dtheta if dtheta.shape == theta_shape else dtheta.view(theta_shape)
 
 
 class E8ThetaWeightQuant(torch.autograd.Function):
@@ -503,11 +503,17 @@ def _aux_stream(device: torch.device) -> "torch.cuda.Stream":
     return s
 
 
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """t as a matrix of its last dimension (itself where it is one: a reshape
+    costs the host as much as an allocation)."""
+    return t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
+
+
 def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: bool):
     """(dx, dW_q, db) of y = x W_q^T + b, None where not needed; bias_dtype is
     None without a bias."""
     need_db = need_db and bias_dtype is not None
-    g2 = gy.reshape(-1, gy.shape[-1])
+    g2, x2 = _rows(gy), _rows(x)
     dx = dW = db = None
     if torch.is_grad_enabled():
         # a backward with create_graph=True: torch's products and sums, which
@@ -515,7 +521,7 @@ def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: b
         if need_dx:
             dx = (g2 @ Wq).reshape(x.shape)
         if need_dw:
-            dW = g2.t() @ x.reshape(-1, x.shape[-1])
+            dW = g2.t() @ x2
         if need_db:
             db = g2.float().sum(0).to(bias_dtype)
         return dx, dW, db
@@ -530,7 +536,6 @@ def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: b
     kernel = None
     fuse = need_dw and fast_db and _FUSE_BIAS_GRAD[0] == 1 and g2.dtype == torch.bfloat16 and g2.is_contiguous()
     if need_dw:
-        x2 = x.reshape(-1, x.shape[-1])
         kernel = _weight_grad_kernel(g2, x2, fuse, need_dx)
         fuse = fuse and kernel is not None
         dbf = torch.empty(g2.shape[1], dtype=torch.float32, device=g2.device) if fuse else None
@@ -564,7 +569,7 @@ def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: b
         dW = weight_grad()
         main.wait_stream(aux)
         if need_dx:
-            dx = dx2.reshape(x.shape)
+            dx = dx2 if x2 is x else dx2.reshape(x.shape)
         if fast_db:
             db = (dbf if fuse else cs[0]).to(bias_dtype)
         elif need_db:
@@ -574,7 +579,9 @@ def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: b
         dW = weight_grad()
         db = dbf.to(bias_dtype)
     if need_dx:
-        dx = (g2 @ Wq).reshape(x.shape)
+        dx = torch.mm(g2, Wq)
+        if x2 is not x:
+            dx = dx.reshape(x.shape)
     if need_dw and not fuse:
         dW = weight_grad()
     if need_db and not fuse:
@@ -638,7 +645,7 @@ class QATLayerFn(torch.autograd.Function):
         Wc = W.detach().contiguous()
         # a bf16 product takes the bias in bf16, written in the launch that writes W_q
         cast = bias is not None and x.dtype == torch.bfloat16
-        Wq, packed, beta, dbdt, b_cast = qat_fwd_theta(Wc, theta.detach(), sigma, xmax, step_count, bounds, q, M, clip,
+        Wq, packed, beta, dbdt, b_cast = qat_fwd_theta(Wc, theta, sigma, xmax, step_count, bounds, q, M, clip,
                                                        bpt, x.dtype, bias if cast else None)
         ctx.save_for_backward(x, Wq, Wc, packed, beta, dbdt)
         ctx.leaves = (W, theta)   # for their place in the graph only: the values are in what is saved
@@ -949,13 +956,13 @@ class HNLQLinearQAT(nn.Module):
         of up to 64 fp32 tokens run as one launch (quantizer and product)."""
         if self._head_takes(x):
             return self._head_forward(x)
+        W, theta = self.weight, self.theta_beta
         if (x.is_cuda and self.quantization_enabled and not self.enable_diagnostics and self._fused()
-                and x.dtype in (torch.float32, torch.bfloat16) and self.weight.is_leaf and self.theta_beta.is_leaf
+                and x.dtype in (torch.float32, torch.bfloat16) and W.is_leaf and theta.is_leaf
                 and getattr(self._quantize_weights_with_bias, "__func__", None) is _QUANTIZE_WEIGHTS):
             self._advance_step(device_increment=False)   # the kernel increments step_count
             bpt = self.blocks_per_row if self.tiling == "row" else 1
-            x = QATLayerFn.apply(x, self.weight, self.theta_beta, self.bias, self.sigma_ema, self.xmax_ema,
-                                 self.step_count,
+            x = QATLayerFn.apply(x, W, theta, self.bias, self.sigma_ema, self.xmax_ema, self.step_count,
                                  ((float(self.Delta0), float(self.eta), self._ginv_f, int(self.M)), int(self.q), 2,
                                   float(self.weight_clip_value), int(bpt)))
             return self.actq(x) if self.quantize_activations and self.actq is not None else x
