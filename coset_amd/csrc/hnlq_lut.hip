@@ -97,6 +97,12 @@ bool lut_path_supported(const CodecArgs& a, int mode)
     if (a.q != 2 && a.q != 4) return false;
     if (a.M < 1 || a.M > 4) return false;
     if (mode == MODE_DECODE && a.codes_in_f32) return false;  // float codes may be off-grid
+    // the words of a block move as one load or store of 4 (M = 2) or 8 (M = 4)
+    // bytes; a view that starts inside one goes to the generic kernel, which
+    // moves each word by itself
+    const uintptr_t words = (uintptr_t)(mode == MODE_DECODE ? a.packed_in : a.packed);
+    const uintptr_t align = a.M == 2 ? 4 : a.M == 4 ? 8 : 2;
+    if (words % align) return false;
     return true;
 }
 

@@ -144,3 +144,26 @@ def test_float_codes_from_the_tile_counter(q, M, n):
         assert torch.equal(a, b)
     assert torch.equal(out[0][0], out[0][2]) and torch.equal(out[0][1], out[0][3])
     assert (out[0][3] >= 0).all() and torch.isfinite(out[0][4]).all()
+
+
+@pytest.mark.parametrize("q,M,skip", [(4, 2, 1), (2, 4, 1), (2, 4, 2), (2, 3, 1), (4, 1, 1)])
+def test_words_that_start_inside_a_load(q, M, skip):
+    """Words at an address that is no multiple of a block's (a view into a
+    larger buffer): decoded, and written through the C ABI, as elsewhere."""
+    import coset_amd as ca
+    from coset_amd import _lib
+    n = (1 << 19) + 5                 # the table kernel's sizes for every mode
+    x = _x(n, 9)
+    words = ca.hnlq_encode(x, q, M, 0.25)
+    buf = torch.zeros(n * M + skip, dtype=torch.int16, device="cuda")
+    buf[skip:] = words.view(torch.int16).reshape(-1)
+    view = buf[skip:].view(n, M)
+    assert view.data_ptr() % (2 * M) != 0 or M == 1 or M == 3
+    for od in (torch.float32, torch.bfloat16):
+        want = ca.hnlq_decode(words, q, M, 0.25, out_dtype=od)
+        assert torch.equal(ca.hnlq_decode(view.view(torch.uint16), q, M, 0.25, out_dtype=od), want)
+    if view.data_ptr() % 4 == 0:      # the entry points take packed words from 4-byte addresses on
+        view.zero_()
+        _lib.call("coset_e8_hnlq_encode", _lib.ptr(x), _lib.F32, n, _lib.SCALE_CODEC, 0.25, None, 0, None, 0, q, M,
+                  view.data_ptr(), None, _lib.stream_of(x))
+        assert torch.equal(view, words.view(torch.int16))
