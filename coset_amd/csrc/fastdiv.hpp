@@ -11,9 +11,12 @@ namespace coset {
 // a / b rounded to nearest even, from y = RN(1/b) (one correctly rounded
 // reciprocal shared by many quotients): q = RN(a y), then STEPS times
 // q <- RN(q + RN(a - b q) y), each a single fused operation.
-// Domain: b, y, a / b and every residual in the normal range -- the callers
-// take 2^-64 <= |b| <= 2^64 and a = 0 or 1/2 <= |a| <= 2^46.  Scaling a and
-// b by powers of two changes nothing there, so take b in [1, 2):
+// Domain: b, y, a / b normal and every residual a multiple of fp32's smallest
+// step.  The residual is one of ulp(b) ulp(q) > 2^-48 |a|, which is at least
+// 2^-149 (subnormals are kept) for |a| >= 2^-100.  The callers take 2^-64 <= |b|
+// <= 2^64 with a = 0 or 1/2 <= |a| <= 2^46, and 2^-20 <= |b| <= 2^20 with 2^-80 <=
+// |a| <= 2^80 (the encoder's dividing betas; STEPS = 2).  Scaling a and b by
+// powers of two changes nothing there, so take b in [1, 2):
 //  - q0 = RN(a y) is within 1.5 ulp of a / b (|y - 1/b| <= 2^-25), so after
 //    the first step, whose residual is a - b q0 to 2^-24 relative, q1 is
 //    within 1/2 ulp + 2^-22 ulp of a / b: a faithful rounding;

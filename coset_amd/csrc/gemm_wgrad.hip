@@ -18,7 +18,7 @@
 // Column sums of A (the bias gradient) come from the same LDS operands: one
 // more MFMA per operand with a first operand of ones, each K stage's by the
 // workgroup of one column tile in turn, so every workgroup adds 1 / tiles_n of
-// them; the partials [splits * tiles_n][M] are added in order.
+// them; the partials [splits * tiles_n][M] are added in order, compensated.
 //
 // Bound: the main loop reaches 1.0 PFLOP/s of the 1.24 a large library product
 // holds on this chip (LDS operand reads and the turning share the issue slots

@@ -3,8 +3,9 @@
 //
 // out[t, o] = s_o sum_k a[t, k] x_hat[o, k] with 2 x_hat held as bytes
 // (VLUT_DECODED, VLUT_DECODED6).  One workgroup of 8 waves per BT tokens x BR
-// rows of the output over the whole K; both operands are staged in LDS, 64 K
-// a stage, double-buffered with one LDS-only barrier per stage:
+// rows of the output and K range (the whole K, or K splits whose partials a
+// reduce adds); both operands are staged in LDS, 64 K a stage, double-buffered
+// with one LDS-only barrier per stage:
 //   activations  [token][8 chunks of 16 bytes], chunk c of token t at
 //                c ^ ((t >> 1) & 7): 16 lanes reading one chunk of 16
 //                consecutive tokens hit 16 distinct 16-byte bank groups;
@@ -12,20 +13,26 @@
 //                fragment order ([row tile][k-quad][lane]), so their stores
 //                and reads are linear.
 // A wave multiplies 16 TT tokens x 16 RT rows: the weights are the MFMA's
-// first operand, so a lane ends with 4 consecutive output rows of one token.  The loads of stage s + 2 go out while stage s is
-// multiplied and their data is stored to LDS in the middle of stage s + 1.
+// first operand, so a lane ends with 4 consecutive output rows of one token.
+// The loads of stage s + 2 go out while stage s is multiplied and their data is
+// stored to LDS in the middle of stage s + 1.
 //
 // fp32 activations (from 43 tokens): one launch and a reduce, where the planes
 // took a split launch, 3B tokens on the deep kernel and a reduce: 197 tokens of
 // 768 x 3072 26.6 -> 17.5 us, 48 of 3072 x 768 13.5 -> 10.6, 4096 of 3072 x 768
-// 306 -> 86; error against 64 bits 6.1e-8 -> 4.6e-8.  At few tokens the time is
-// the latency of the stages (0.9 us each, 64 x 64 tiles) and of the reduce.
+// 306 -> 86; error against 64 bits (197 of 768 x 3072) 5.8e-8 -> 3.9e-8.  At few
+// tokens the time is the latency of the stages (0.9 us each, 64 x 64 tiles) and
+// of the reduce.
 //
-// Bound: at 4096 x 4096 x 4096 tokens 1148 TFLOP/s (bf16, 256 x 256 tiles over the whole K), the matrix cores at
-// the clock the chip holds under them; at 3072 x 768 x 4096 tokens 38 us on the plan's
-// 128 x 128 tiles (kOneChainK), of which the 50 MB of fp32 output take 10 (the deep
-// kernel, which decodes each weight for 64 tokens, takes 104).  Decoding at the store to LDS costs one
-// decode per BT tokens, 20 VALU operations per 8 weights in bf16.  Waves in
+// Bound: at 3072 x 768 x 4096 tokens 38 us on the plan's 128 x 128 tiles, three
+// rounds of 256 (the deep kernel, which decodes each weight for 64 tokens, takes
+// 104): 464 TFLOP/s in a kernel trace, no LDS bank conflicts, the matrix cores
+// busy about a fifth of the time; the rest is the wait for a stage's operands, its
+// decode and, last in each round, the stores of 50 MB of fp32 output (10 us).
+// The 256 x 256 tiles, forced at 4096 x 4096 x 4096 tokens, reach 1148 TFLOP/s, but
+// the plan takes the 256-token tiles up to kOneChainK only.  Decoding at the
+// store to LDS costs one decode per BT tokens (128 above kOneChainK), 20 VALU
+// operations per 8 weights in bf16.  Waves in
 // two groups a phase apart (one loads while the other multiplies) measured the
 // same at full load and slower on the smaller shapes; 4 waves of 128 x 128
 // do not fit the registers.
@@ -188,7 +195,8 @@ __global__ void __launch_bounds__(WT * WR * 64) vlut_gemm_kernel(VlutMatmulArgs 
     // kTwo: sums in two steps -- every 256 K the products' accumulator is added to
     // a total and cleared -- so the error stays that of the deep kernel's short
     // chains (768 x 3072 fp32: 6.1e-8 against 64 bits, 7.8e-8 in one chain).  The
-    // 256-token shapes have no registers for it; the plan gives them up to 1024 K.
+    // 256-token shapes have no registers for it; the plan gives them up to
+    // kOneChainK.
     constexpr bool kTwo = A32 || RT * TT <= 8;
     constexpr int NA = A32 ? 2 : 1;
     float4_t acc[RT][NA * TT];   // token tile t; A32: the lower planes at TT + t
@@ -349,7 +357,9 @@ struct GemmShape {
 // The most K that the 256-token tiles, whose sums are one chain, take: above,
 // their error against 64 bits is larger than the deep kernel's (fp16, 1000 K
 // 7.7e-8 against 6.7e-8, 128 x 128 tiles 6.5e-8; bf16, 768 K 5.1e-8, 5.0e-8,
-// 5.0e-8), though 4096 tokens of 3072 x 768 take 29 us on them and 38 on 128 x 128
+// 5.0e-8), though 4096 tokens of 3072 x 768 take 29 us on them and 38 on 128 x
+// 128.  Up to it they serve large outputs: 8192 tokens of 8192 x 256 77 us against
+// 100 on 128 x 128 tiles, 16384 of 4096 x 128 63 / 85, 8192 of 3072 x 256 32 / 37
 constexpr int64_t kOneChainK = 256;
 constexpr GemmShape kGemmShapes[] = {{256, 256, 1.51, 8.3}, {256, 192, 1.26, 8.1}, {128, 128, 0.59, 4.1},
                                      {128, 64, 0.43, 3.5}};

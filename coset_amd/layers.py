@@ -549,7 +549,7 @@ def linear_grads(gy, x, Wq, bias_dtype, need_dx: bool, need_dw: bool, need_db: b
         return out
 
     if overlap:
-        # dX (and the bias gradient where no weight-gradient kernel takes it)
+        # dX (and the bias gradient where torch.mm computes dW)
         # on a second stream while dW runs on this one: the dW product
         # alone leaves CUs idle at these shapes (one 64 x 64 or 128 x 128
         # tile per CU or fewer).  Outputs are allocated here, on the

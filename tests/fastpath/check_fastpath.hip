@@ -34,7 +34,7 @@
 //                                   significand in [1, 2) and a = k / 2,
 //                                   k = 0 .. K (signs of a and b varied),
 //                                   plus, for S >= 2, random a of any
-//                                   exponent in the helper's domain
+//                                   exponent in its callers' domains
 //   check_fastpath u32div N         u32div against n / d: every d < 2^16 and
 //                                   N random d, each with the n next to its
 //                                   multiples, the ends of the range and
@@ -376,7 +376,8 @@ static int fast_residual(long n, int threads)
 // [1, 2) (the quotient's rounding does not depend on b's exponent in the
 // helper's domain), a = k / 2 for k = 0 .. K with the four sign pairs on
 // every 16th b, and for S >= 2 eight random a per b with exponents from
-// 2^-1 to 2^46 and b scaled by 2^-64 .. 2^64
+// 2^-1 to 2^46 and b scaled by 2^-64 .. 2^64, and eight with 2^-80 <= |a| < 2^80
+// and 2^-20 <= |b| < 2^20 (the encoder's dividing betas)
 template <int S>
 static int divq(long K, int threads)
 {
@@ -421,6 +422,12 @@ static int divq(long K, int threads)
                         const float a = ldexpf(from_bits(0x3f800000u | (uint32_t)(h >> 40 & 0x7fffff)), ea);
                         const float bb = ldexpf(b, eb), yy = ldexpf(y, -eb);
                         check((h >> 63) ? -a : a, bb, yy);
+                    }
+                    for (int t = 0; t < 8; ++t) {
+                        const uint64_t h = g();
+                        const int ea = (int)(h % 160) - 80, eb = (int)((h >> 8) % 40) - 20;
+                        const float a = ldexpf(from_bits(0x3f800000u | (uint32_t)(h >> 40 & 0x7fffff)), ea);
+                        check((h >> 63) ? -a : a, ldexpf(b, eb), ldexpf(y, -eb));
                     }
                 }
             }
