@@ -23,6 +23,7 @@
 #include <stdint.h>
 
 #include "e8_fast.hpp"
+#include "rounding.hpp"
 
 namespace coset {
 
@@ -308,15 +309,6 @@ __device__ __forceinline__ void add_level(float acc[8], float w, const float r[8
 __device__ __forceinline__ float bf16_to_f32(uint16_t h)
 {
     return __uint_as_float(((uint32_t)h) << 16);
-}
-
-// fp32 -> bf16 round-to-nearest-even (NaN kept quiet).
-__device__ __forceinline__ uint16_t f32_to_bf16(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
 }
 
 }  // namespace coset

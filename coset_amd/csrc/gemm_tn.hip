@@ -34,6 +34,7 @@
 #include <utility>
 
 #include "gemm.hpp"
+#include "rounding.hpp"
 
 namespace coset {
 namespace {
@@ -78,14 +79,6 @@ __device__ __forceinline__ void unroll_steps(F& f, int s0, std::integer_sequence
     (f(s0 + I, std::integral_constant<int, I>{}), ...);
 }
 
-__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);   // NaN stays a (quiet) NaN
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-
 // 8 consecutive outputs: fp32 (OUT 0, 2) or bf16 (OUT 1)
 template <int OUT>
 __device__ __forceinline__ void store8(void* C, int64_t idx, const float v[8])
@@ -94,7 +87,7 @@ __device__ __forceinline__ void store8(void* C, int64_t idx, const float v[8])
         uint32_t h[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            h[q] = (uint32_t)f32_to_bf16_rne(v[2 * q]) | ((uint32_t)f32_to_bf16_rne(v[2 * q + 1]) << 16);
+            h[q] = pack_bf16(v[2 * q], v[2 * q + 1]);
         *reinterpret_cast<uint4*>(static_cast<uint16_t*>(C) + idx) = make_uint4(h[0], h[1], h[2], h[3]);
     } else {
         float4* dst = reinterpret_cast<float4*>(static_cast<float*>(C) + idx);

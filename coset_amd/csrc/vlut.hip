@@ -623,16 +623,6 @@ __global__ void __launch_bounds__(256) vlut_reduce_kernel(const float* partial, 
     out[i] = vlut_epilogue(acc * mult * sc, o, bias, lsq_alpha, lsq_qmax);
 }
 
-// acc + low <- acc + low + w with the rounding error of acc + w kept in low
-// (Knuth's two-sum); a sum that is not finite leaves low not finite, and the
-// callers then drop it
-__device__ __forceinline__ void two_sum(float& acc, float& low, float w)
-{
-    const float t = __fadd_rn(acc, w), b = __fsub_rn(t, acc);
-    low = __fadd_rn(low, __fadd_rn(__fsub_rn(acc, __fsub_rn(t, b)), __fsub_rn(w, b)));
-    acc = t;
-}
-
 // Same for partials stored split-major, [splits][B][rows] (the wide kernel);
 // the splits are summed in order.
 // COMP: compensated, for the GEMM kernel's many splits (below).
@@ -653,7 +643,7 @@ __global__ void __launch_bounds__(256) vlut_reduce_sm_kernel(const float* partia
         else
             acc += partial[s * n + i];
     }
-    if (COMP && low - low == 0.f) acc = __fadd_rn(acc, low);
+    if (COMP) acc = two_sum_value(acc, low);
     float sc = scale ? (scale_mode == 0 ? scale[o] : 1.f / scale[o]) : 1.f;
     out[i] = vlut_epilogue(acc * mult * sc, o, bias, lsq_alpha, lsq_qmax);
 }
@@ -725,8 +715,7 @@ __global__ void __launch_bounds__(256) vlut_reduce_rg4_kernel(const float* parti
     }
     if constexpr (COMP) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (low[j] - low[j] == 0.f) acc[j] = __fadd_rn(acc[j], low[j]);
+        for (int j = 0; j < 4; ++j) acc[j] = two_sum_value(acc[j], low[j]);
     }
     float r[4];
 #pragma unroll
