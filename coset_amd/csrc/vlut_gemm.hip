@@ -361,7 +361,7 @@ struct GemmShape {
 // 128.  Up to it they serve large outputs: 8192 tokens of 8192 x 256 77 us against
 // 100 on 128 x 128 tiles, 16384 of 4096 x 128 63 / 85, 8192 of 3072 x 256 32 / 37
 constexpr int64_t kOneChainK = 256;
-constexpr GemmShape kGemmShapes[] = {{256, 256, 1.51, 8.3}, {256, 192, 1.26, 8.1}, {128, 128, 0.59, 4.1},
+constexpr GemmShape kGemmShapes[] = {{256, 256, 1.51, 8.3}, {256, 192, 1.26, 8.1}, {128, 128, 0.61, 4.1},
                                      {128, 64, 0.43, 3.5}};
 
 constexpr GemmShape kGemmShapes32[] = {{128, 128, 1.98, 4.3}, {64, 128, 1.1, 3.7}, {64, 64, 0.9, 3.3}};
@@ -434,22 +434,24 @@ VlutPlan vlut_gemm_plan(int64_t rows, int64_t B, int64_t K, int cus)
     // 4096 x 4096: 10.8 us against 31)
     if (B <= 2 * kDeepTokens - 1) return none;
     // the deep kernel: 64 x 64 tiles of at most 1024 K, 7.2 us a round of one
-    // workgroup per CU (its phases do not overlap).  The reduce of its splits
-    // takes 0.8 us where each XCD reads the partials its own workgroups wrote
-    // (rows a multiple of 8 groups of 64), else 2.0.  With these costs the choice
-    // is within 2.5 % of the faster kernel at 517 of 520 measured calls (20 shapes
-    // of 512..4096 x 320..4096, 128 to 2000 tokens, bf16 and fp16; the worst 4.5 %
-    // off).  bf16, us, deep / this kernel: 768 x 3072 x 160 tokens (the splits fill
-    // the chip) 11.4 / 12.4, x 512 18.4 / 15.6, x 1024 28.5 / 20.3; 2048 x 1000 x 160
-    // 9.7 / 10.6; 768 x 768 x 160 11.3 / 8.7; 3072 x 768 x 4096 103.9 / 38.1; 4096 x
-    // 4096 x 256 34.3 / 22.5, x 4096 557 / 157 on 128 x 128 tiles (120 on 256 x 256,
-    // which sum 4096 K in one chain)
+    // workgroup per CU (its phases do not overlap), and every XCD reads the
+    // activations, which few rows of many tokens wait for (2000 tokens of 512 x 2048
+    // 25 us, two rounds; this kernel 18.5).  The reduce of its splits takes 0.8 us
+    // where each XCD reads the partials its own workgroups wrote (rows a multiple of
+    // 8 groups of 64), else 2.0.  With these costs the choice is within 2.5 % of the
+    // faster kernel at all but 8 of 806 measured calls (256..4096 x 256..4096, 128 to
+    // 8192 tokens, bf16 and fp16; the worst 10 % off).  bf16, us, deep / this
+    // kernel: 768 x 3072 x 160 tokens (the splits fill the chip) 11.4 / 12.4, x 512
+    // 18.4 / 15.6, x 1024 28.5 / 20.3; 2048 x 1000 x 160 9.7 / 10.6; 768 x 768 x 160
+    // 11.3 / 8.7; 3072 x 768 x 4096 103.9 / 38.1; 4096 x 4096 x 256 34.3 / 22.5, x 4096
+    // 557 / 157 on 128 x 128 tiles (120 on 256 x 256, which sum 4096 K in one chain)
     const int64_t kq = (K / 8 + 3) / 4;
     const int64_t groups = ((rows + kDeepRows - 1) / kDeepRows) * ((B + kDeepTokens - 1) / kDeepTokens);
     const int64_t min_splits = (kq + kDeepKqWg - 1) / kDeepKqWg;
     const int64_t splits = std::max(min_splits, std::min<int64_t>(std::max<int64_t>(1, cus / groups), kq));
     const double reduce_us = splits == 1 ? 0.0 : rows % (8 * kDeepRows) == 0 ? 0.8 : 2.0;
-    const double deep_us = 1.4 + 7.2 * (double)((groups * splits + cus - 1) / cus) + reduce_us;
+    const double reads_us = 8.0 * (double)(B * K) * 2.0 / 33.0e6;
+    const double deep_us = 1.3 + 7.2 * (double)((groups * splits + cus - 1) / cus) + reads_us + reduce_us;
     // workspaces are sized for the deep plan's splits
     VlutPlan best;
     return best_gemm(kGemmShapes, 4.5, rows, B, K, cus, splits, &best) < deep_us ? best : none;
