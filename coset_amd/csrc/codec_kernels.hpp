@@ -180,12 +180,8 @@ extern int g_codec_plain;      // 1 (default): the table kernel's fixed-format v
 extern int g_codec_dynamic;    // 1 (default): the fixed-format kernel takes its tiles from a counter
 // The fixed-format variant of the table kernel takes this call (q = 2, 4).
 bool lut_plain_supported(const CodecArgs& a, int mode);
-// Blocks from which the table kernel is used (below, its table staging does
-// not pay): the fixed-format variant's (encode and decode, round trip), and the
-// general one's.  q4 M2, fp32, us, generic / table: decode of 2^17 blocks 4.6 /
-// 4.7, of 2^18 6.3 / 5.5 (bf16 rows 6.1 / 4.9), encode of 2^18 5.7 / 5.3, round
-// trip of 2^18 8.2 / 7.5 unscaled but 7.6 / 7.7 by rows, of 2^19 13.2 / 10.7.
-constexpr int64_t kLutMinBlocksPlain = 1 << 18, kLutMinBlocksPlainRt = 1 << 19, kLutMinBlocks = 1 << 20;
+// Whether the table kernels are the faster ones for a call they support.
+bool lut_pays(const CodecArgs& a, int mode);
 // A zeroed counter pair of the current device's counter ring (counters.hpp)
 // for one launch on stream s, held until the launch's last workgroup puts the
 // pair back to zero and stores 1 to *release; pair is null (static schedule)

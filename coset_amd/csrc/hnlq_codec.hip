@@ -712,11 +712,10 @@ hipError_t launch_codec(const CodecArgs& args, int mode, hipStream_t s)
     a.fast_projection = g_fast_projection;
     // the general table kernel leaves the layer quantizer with betas from
     // theta to the layer round-trip kernel (3072 x 3072 to bf16: 33.5 -> 22.6 us)
-    const bool plain = lut_plain_supported(a, mode);
-    const int64_t from = !plain ? kLutMinBlocks : mode == MODE_ROUNDTRIP ? kLutMinBlocksPlainRt : kLutMinBlocksPlain;
     const bool lut = lut_path_supported(a, mode) &&
                      (g_codec_path == 2 ||
-                      (g_codec_path == 0 && a.n >= from && (plain || !layer_rt_supported(a, mode, true))));
+                      (g_codec_path == 0 && lut_pays(a, mode) &&
+                       (lut_plain_supported(a, mode) || !layer_rt_supported(a, mode, true))));
     if (a.aux_out && a.aux_n > 0 && (lut || a.n == 0)) {
         // the table kernels take no side cast: it gets its own launch
         hipLaunchKernelGGL(aux_cast_kernel, dim3((unsigned)((a.aux_n + 255) / 256)), dim3(256), 0, s, a);

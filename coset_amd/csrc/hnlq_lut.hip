@@ -135,6 +135,32 @@ bool lut_plain_supported(const CodecArgs& a, int mode)
     return true;
 }
 
+// From 2^20 blocks on always (below, the general kernel's table staging does
+// not pay).  The fixed-format kernel starts earlier: its decode at 2^18 blocks
+// (q4 M2 fp32, us, generic / table: 2^17 4.6 / 4.7, 2^18 6.3 / 5.5), its fp32 round
+// trip at 2^19 (2^18 8.2 / 7.5 unscaled but 7.6 / 7.7 by rows, 2^19 13.2 / 10.7), float
+// codes of two levels at 2^18 (10.9 / 7.9).  The other encoders and round trips
+// are bound by their arithmetic, which one workgroup of 1024 threads per CU
+// spreads in whole rounds of 2^18 blocks and the generic kernel in small ones:
+// they take the table kernel where the last round is full to nine tenths of all
+// (encode q4 M2 by rows in bf16: 300000 blocks 7.1 / 8.2, 2^19 9.4 / 9.3, 800000 12.0 /
+// 13.4, 10^6 13.8 / 13.7; round trip unscaled in bf16, q4 M1: 600000 blocks 10.6 /
+// 12.7), and never where bf16 values come unscaled or by 2^k, whose ties the
+// generic encoder resolves faster (2^19 blocks q4 M1 8.8 / 9.7).
+bool lut_pays(const CodecArgs& a, int mode)
+{
+    if (a.n >= (1 << 20)) return true;
+    if (!lut_plain_supported(a, mode) || a.n < (mode == MODE_ROUNDTRIP ? 1 << 19 : 1 << 18)) return false;
+    const bool layer = a.scale_mode == SCALE_LAYER;
+    const bool bf = (mode != MODE_DECODE && a.x_dtype == DT_BF16) || (mode != MODE_ENCODE && a.out_dtype == DT_BF16);
+    if (mode == MODE_DECODE) return true;
+    if (mode == MODE_ROUNDTRIP && (layer ? a.q == 2 : !bf)) return true;   // by rows at q = 4: the layer kernel
+    if (mode == MODE_ENCODE && a.codes_f32 && a.M == 2) return true;
+    if (mode == MODE_ENCODE && bf && !layer && (a.scale_mode != SCALE_CODEC || a.beta_is_pow2)) return false;
+    const int64_t round = (int64_t)cu_count() * kLutThreads, rounds = (a.n + round - 1) / round;
+    return 10 * a.n >= 9 * rounds * round;
+}
+
 hipError_t launch_codec_lut(const CodecArgs& a, int mode, hipStream_t s)
 {
     const DecodeTables* t = nullptr;

@@ -167,3 +167,33 @@ def test_words_that_start_inside_a_load(q, M, skip):
         _lib.call("coset_e8_hnlq_encode", _lib.ptr(x), _lib.F32, n, _lib.SCALE_CODEC, 0.25, None, 0, None, 0, q, M,
                   view.data_ptr(), None, _lib.stream_of(x))
         assert torch.equal(view, words.view(torch.int16))
+
+
+@pytest.mark.parametrize("op,n,q,M,dt,beta,table", [
+    ("encode", 300000, 4, 2, torch.float32, 0.25, False), ("encode", 300000, 4, 1, torch.bfloat16, "row", False),
+    ("encode", 1 << 19, 4, 2, torch.float32, 0.3, True), ("encode", 1 << 19, 4, 2, torch.bfloat16, None, False),
+    ("encode", 800000, 4, 1, torch.bfloat16, None, False), ("encode", (1 << 20) + 8, 4, 2, torch.bfloat16, None, True),
+    ("roundtrip", 600000, 4, 1, torch.bfloat16, None, False), ("roundtrip", 600000, 4, 2, torch.float32, 0.3, True),
+    ("roundtrip", 600000, 2, 3, torch.float32, "row", True), ("decode", 300000, 4, 2, torch.bfloat16, "row", True),
+    ("decode", 200000, 4, 2, torch.float32, None, False)])
+def test_kernel_of_a_call(op, n, q, M, dt, beta, table):
+    """Which kernel takes a call of 2^18 to 2^20 blocks (both give the same
+    bits): the names a profiler sees."""
+    from torch.profiler import ProfilerActivity, profile
+    import coset_amd as ca
+    n = n // 8 * 8
+    x = torch.randn(n, 8, device="cuda").to(dt)
+    kw = dict(beta=beta)
+    if beta == "row":
+        kw = dict(beta_row=torch.rand(n // 8, device="cuda") + 0.5, blocks_per_row=8)
+    words = ca.hnlq_encode(x, q, M, **kw)
+    fn = {"encode": lambda: ca.hnlq_encode(x, q, M, **kw), "roundtrip": lambda: ca.hnlq_roundtrip(x, q, M, **kw),
+          "decode": lambda: ca.hnlq_decode(words, q, M, out_dtype=dt, **kw)}[op]
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        fn()
+        torch.cuda.synchronize()
+    names = [e.key for e in p.key_averages()]
+    assert any("hnlq" in k for k in names), names
+    assert any("hnlq_plain_kernel" in k or "hnlq_lut_kernel" in k for k in names) == table, names
