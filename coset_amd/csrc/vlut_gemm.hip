@@ -439,10 +439,14 @@ VlutPlan vlut_gemm_plan(int64_t rows, int64_t B, int64_t K, int cus)
     // 25 us, two rounds; this kernel 18.5).  The reduce of its splits takes 0.8 us
     // where each XCD reads the partials its own workgroups wrote (rows a multiple of
     // 8 groups of 64), else 2.0.  With these costs the choice is within 2.5 % of the
-    // faster kernel at all but 8 of 806 measured calls (256..4096 x 256..4096, 128 to
-    // 8192 tokens, bf16 and fp16; the worst 10 % off).  bf16, us, deep / this
-    // kernel: 768 x 3072 x 160 tokens (the splits fill the chip) 11.4 / 12.4, x 512
-    // 18.4 / 15.6, x 1024 28.5 / 20.3; 2048 x 1000 x 160 9.7 / 10.6; 768 x 768 x 160
+    // faster kernel at all but 8 of 806 measured calls replayed from a graph
+    // (256..4096 x 256..4096, 128 to 8192 tokens, bf16 and fp16; the worst 10 % off).
+    // A split deep call is charged 1.5 us more against an unsplit one of this kernel:
+    // an eager call waits for the host, which takes 14 us for two launches and 9.5
+    // for one.  That decides 40 of the calls, by up to 15 % for the slower kernel
+    // in a graph and 26 % for the faster one outside (2048 x 1000 x 160: 9.7 / 10.6).
+    // bf16, us, deep / this kernel, in a graph: 768 x 3072 x 160 tokens (the splits
+    // fill the chip) 11.4 / 12.4, x 512 18.4 / 15.6, x 1024 28.5 / 20.3; 768 x 768 x 160
     // 11.3 / 8.7; 3072 x 768 x 4096 103.9 / 38.1; 4096 x 4096 x 256 34.3 / 22.5, x 4096
     // 557 / 157 on 128 x 128 tiles (120 on 256 x 256, which sum 4096 K in one chain)
     const int64_t kq = (K / 8 + 3) / 4;
@@ -454,7 +458,8 @@ VlutPlan vlut_gemm_plan(int64_t rows, int64_t B, int64_t K, int cus)
     const double deep_us = 1.3 + 7.2 * (double)((groups * splits + cus - 1) / cus) + reads_us + reduce_us;
     // workspaces are sized for the deep plan's splits
     VlutPlan best;
-    return best_gemm(kGemmShapes, 4.5, rows, B, K, cus, splits, &best) < deep_us ? best : none;
+    const double us = best_gemm(kGemmShapes, 4.5, rows, B, K, cus, splits, &best);
+    return us < deep_us + (splits > 1 && best.splits == 1 ? 1.5 : 0.0) ? best : none;
 }
 
 VlutPlan vlut_gemm32_plan(int64_t rows, int64_t B, int64_t K, int cus, int64_t max_splits)

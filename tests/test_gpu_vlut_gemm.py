@@ -189,13 +189,13 @@ def test_fp32_at_the_gemm_kernels_first_tokens(layout, rows, K):
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("B,rows,K,shape", [(127, 768, 768, None), (160, 768, 3072, None), (129, 2048, 1000, None),
+@pytest.mark.parametrize("B,rows,K,shape", [(127, 768, 768, None), (160, 768, 3072, None), (129, 2048, 1000, 3),
                                             (160, 3072, 3072, None), (256, 768, 2048, None), (256, 256, 256, 3),
                                             (512, 3072, 768, 3), (1000, 3072, 768, 2), (4096, 512, 512, 2),
                                             (2000, 512, 2048, -1), (700, 4096, 4096, -1)])
 def test_plan_takes_the_faster_kernel(dt, B, rows, K, shape):
     """Where the deep kernel is the faster one (its splits fill the chip in one
-    round) the plan takes it, else this kernel in the named shape (-1: with K
+    round, and no unsplit launch is about as fast) the plan takes it, else this kernel in the named shape (-1: with K
     splits): told apart by the bits of the sums, which the two add in different
     orders."""
     import coset_amd as ca
